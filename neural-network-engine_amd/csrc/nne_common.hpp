@@ -15,8 +15,56 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 // which can keep register arrays of it out of registers.)
 typedef float vf4 __attribute__((ext_vector_type(4)));
 
+// Operand of a bf16 MFMA: 8 values of one lane.
+typedef short short8 __attribute__((ext_vector_type(8)));
+typedef float vf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegInf = -__builtin_huge_valf();
+
+// ---- f32 products on the bf16 matrix cores -----------------------------------
+// An f32 value is the exact sum of three bf16 values (8 significant bits and a
+// sign each, rounded to nearest: 24 bits in all), and the product of two of
+// them is nine bf16 products.  The six largest are computed,
+//   xy = hh + (hm + mh) + (mm + hl + lh) + O(2^-25 |xy|),
+// each product exact and every sum in f32, as on the f32 MFMAs; with h, m and
+// l the high, middle and low parts.  gfx950's bf16 MFMAs run at 16x the rate
+// of its f32 ones, so six of them take 3/8 of the time (measured on registers:
+// 1777 / 6 = 296 against 146 TFLOP/s), and their sums are rounded less often:
+// the error of a 128-term dot product of N(0, 1) values against 64 bits is
+// 0.7e-7 to 1.6e-7 (two accumulators, one) where the f32 MFMAs give 2.0e-7.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(vf2{a, b}, bf16x2));
+}
+// The three parts of a (low 16 bits) and b (high 16 bits).
+__device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = pack_bf16(a, b);
+    a -= __uint_as_float(h << 16);
+    b -= __uint_as_float(h & 0xffff0000u);
+    m = pack_bf16(a, b);
+    a -= __uint_as_float(m << 16);
+    b -= __uint_as_float(m & 0xffff0000u);
+    l = pack_bf16(a, b);
+}
+__device__ __forceinline__ floatx16 mfma_bf16(short8 a, short8 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+// Where the parts do not hold a value: an infinity, a NaN or a magnitude that
+// rounds to infinity leaves NaN parts, and every result it enters is NaN; below
+// 2^-100 the low parts fall under bf16's normal range, which the MFMAs flush.
+// Results show both (a tiny V gives tiny O), except where a tiny query meets a
+// huge key or a huge query a tiny key, so queries have a range of their own.
+// (range_code: 0 for zero, ascending with the magnitude from 2^-90 on, above
+// every such code for smaller magnitudes.)
+__device__ __forceinline__ uint32_t range_code(float x) {
+    const uint32_t a = __float_as_uint(x) & 0x7fffffffu;
+    return a == 0 ? 0 : a - __float_as_uint(0x1p-90f);
+}
+constexpr uint32_t kResultCodes = 0x7f800000u - 0x12800000u;   // codes of finite results
+constexpr uint32_t kQueryCodes = 0x6c800000u - 0x12800000u;    // codes of queries up to 2^90
 
 // Brings [B0, E0) and [B1, E1) of the kernel argument block into the scalar
 // cache: one load per 64-byte line, all issued before a single wait.  The

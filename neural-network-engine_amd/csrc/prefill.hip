@@ -1,4 +1,4 @@
-// FlashAttention forward for gfx950 on full-fp32 MFMA (v_mfma_f32_32x32x2_f32).
+// FlashAttention forward for gfx950: f32 on the bf16 matrix cores.
 //
 // Algorithm: the tiled online softmax of the reference's
 // flash_attention_forward (src/nn/flash_attention.rs:91-195) -- per query row a
@@ -7,29 +7,43 @@
 // skipped (:101-104) -- generalised to grouped-query heads (KV head hq / G) and
 // a causal offset.
 //
-// MI355X mapping.  One wave owns 32 query rows and computes the score tile
-// transposed, S^T = K Q^T, on 32x32x2 MFMAs:
-//   A = K tile  (lane l supplies key l%32, reduction index l/32)
+// MI355X mapping (head dims up to 128; 129-256 dims: prefill_wide_kernel).
+// Every f32 operand is the exact sum of three bf16 parts and every product the
+// six largest products of parts (nne_common.hpp), on v_mfma_f32_32x32x16_bf16.
+// One wave owns 32 query rows and computes the score tile transposed,
+// S^T = K Q^T:
+//   A = K tile  (lane l supplies key l%32, dims 16t + 8*(l/32) + 0..7 of step t)
 //   B = Q^T     (lane l supplies query row l%32; held in registers, pre-scaled
 //                by scale*log2(e) so the softmax is a bare exp2)
-// The reduction (head-dim) order is permuted so that lane half h covers dims
-// [h*D/2, h*D/2 + D/2): each lane then reads its K operands as contiguous
-// 16-byte LDS vectors.  The accumulator layout of S^T puts query row l%32 in
-// lane l and keys 8*(r/4) + 4*(l/32) + r%4 in register r, so
+// The accumulator layout of S^T puts query row l%32 in lane l and keys
+// 8*(r/4) + 4*(l/32) + r%4 in register r, so
 //   * the row max / row sum are 16 in-lane ops plus one lane-pair exchange
 //     (v_permlane32_swap),
-//   * P^T register r is already the B operand of step r of O^T = V^T P^T
-//     (the key order of that reduction is chosen to match), so P never
-//     leaves registers,
+//   * the parts of P^T registers 8s .. 8s + 7 are already the B operand of step
+//     s of O^T = V^T P^T (V's keys are laid out to match), so P never leaves
+//     registers,
 //   * every O^T accumulator of a lane belongs to that lane's query row, so the
 //     online-softmax rescale is a lane-local multiply -- done lazily, only
 //     when a row max grows by more than 2^8.
-// K and V tiles (32 keys) are staged through LDS, double buffered, with the
-// next tile's global loads in flight while the current tile is computed.  The
-// G query heads that share a KV head run as waves of one workgroup and read
-// the same staged tiles.  Workgroups are numbered so that each XCD works on a
-// contiguous range of KV heads (its own L2) and, within a head, the longest
-// causal row blocks start first.
+// K and V tiles (32 keys) are split into their parts by the threads that load
+// them, once per workgroup, and left in LDS in operand order: 6 bytes a value.
+// One buffer each for K and V: a tile's K is replaced while its softmax and
+// P V run, its V while the next S^T runs, each from registers loaded a phase
+// before, with a barrier between the phases; at D = 128 two workgroups (49 KB
+// of tiles each) share a CU and fill each other's waits.  The G query heads
+// that share a KV head run as waves of one workgroup and read the same staged
+// tiles.  Workgroups are numbered so that each XCD works on a contiguous range
+// of KV heads (its own L2) and, within a head, the longest causal row blocks
+// start first.
+//
+// What bounds it: the matrix cores, and the power they draw.  A tile takes a
+// wave 96 MFMAs of 32 cycles at D = 128 beside about 340 vector instructions
+// (softmax, the parts of P, K and V); with random operands a stream of nothing
+// but these MFMAs settles at 1777 TFLOP/s, 296 TFLOP/s of f32 products.
+// Measured against the f32 MFMAs (v_mfma_f32_32x32x2, 157 TFLOP/s at most):
+// B = 4, Hq = 32, Hkv = 8, T = 2048, d = 128 causal 1067 -> 742 us, B = 1,
+// H = 16, T = 16384, d = 64 causal 4300 -> 2800 us, B = 8, H = 20, T = 1500,
+// d = 64 774 -> 475 us, with 0.6 to 0.9 of the error against 64 bits.
 //
 // Problems with fewer work items than CUs instead cut each item's key tiles
 // into chunks, one workgroup per (item, chunk); the last chunk of an item to
@@ -144,17 +158,251 @@ __device__ __forceinline__ int item_at(const PrefillParams& p, int j, int x, int
     return 1;
 }
 
-// Two workgroups per CU for the persistent schedule.  At d = 128 the
-// key-split variant (small problems, one short chunk per workgroup) and the
-// scalar-load variant (views that are not 16-byte vectors) take the whole
-// register file instead of spilling.
+// K/V tile of 32 keys x D dims, read by 256 threads and left in LDS as three
+// bf16 planes each, in operand order (one 16-byte slot per lane):
+//   K (A of S^T = K Q^T): plane p, 16-dim step t, lane half h, key r at slot
+//     (p * D/16 + t) * 64 + h * 32 + (r ^ ((2t + h) & 15)), dims 16t + 8h .. + 7.
+//     The XOR spreads the 16 slots that one key's dims are stored to over the
+//     banks; a step's reads stay one contiguous 1 KB.
+//   V (A of O^T = V^T P^T): plane p, 32-dim block b, 16-key step s, lane half
+//     h, dim m at slot ((p * NB + b) * 2 + s) * 64 + h * 32 + m, keys
+//     16s + 4h + 0..3 and 16s + 8 + 4h + 0..3 (the keys of lane half h in
+//     registers 8s .. 8s + 7 of the S^T accumulator).
+// Rows past T_k are zeros, or with scalar loads row T_k - 1 again (their
+// weights are zero); dims past d read dim 0 (Q is zero there, and those output
+// dims are not stored).
+template <int D, bool VEC>
+struct SplitTile {
+    static constexpr int NB = D / 32;
+    static constexpr int K_PLANE = 32 * D * 2, V_PLANE = 32 * D * 2;   // bytes
+    static constexpr int LPR = D / 4;                // lanes per key row (4 dims each)
+    static constexpr int RPI = 64 / LPR;             // rows per load
+    static constexpr int NK = 8 / RPI;               // K loads per thread
+    static_assert(64 % LPR == 0 && 8 % RPI == 0, "whole rows per load");
+    static constexpr int NJ = (D + 63) / 64;         // dims per lane of V
+    float4 kr[NK];
+    float vr[NJ][8];
+    // VEC views (row strides in [0, 2^24)): byte offsets of this lane within a
+    // tile and of each load's rows, so that a tile's loads need only its base.
+    uint32_t k_lane, k_step, v_lane[NJ], v_row0, v_st;
+
+    __device__ __forceinline__ void init(const PrefillParams& p, int wave, int lane) {
+        const int c = (lane % LPR) * 4;
+        const uint32_t kst = (uint32_t)p.k.st * 4u, vst = (uint32_t)p.v.st * 4u;
+        k_lane = (8 * wave + lane / LPR) * kst + (c < p.d ? c : 0) * 4;
+        k_step = RPI * kst;
+        v_row0 = (16 * (wave >> 1) + 4 * (wave & 1)) * vst;
+        v_st = vst;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) v_lane[j] = (lane + 64 * j < p.d ? lane + 64 * j : 0) * 4;
+    }
+
+    // Rows key0 .. key0 + 31 of a KV head, ending with the last key (rows past
+    // it read as zeros without a memory access).
+    // (Without a tile, ok false: an empty range.)
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_range(const float* base, int64_t st,
+                                                                        int key0, int Tk, int d, bool ok) {
+        const int rows = min(32, Tk - key0);
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(base + key0 * st), 0,
+            ok ? ((rows - 1) * (uint32_t)st + d) * 4u : 0u, 0x00020000);
+    }
+
+    __device__ __forceinline__ void load_k(const PrefillParams& p, const float* kb, int key0,
+                                           int wave, int lane, bool ok) {
+        if (VEC) {
+            const auto range = tile_range(kb, p.k.st, key0, p.Tk, p.d, ok);
+            if (ok && key0 + 32 <= p.Tk) {
+#pragma unroll
+                for (int i = 0; i < NK; ++i)
+                    kr[i] = __builtin_bit_cast(
+                        float4, __builtin_amdgcn_raw_buffer_load_b128(range, k_lane, i * k_step, 0));
+            } else {
+                // The range check is on the lane's offset, so all of it goes there.
+#pragma unroll
+                for (int i = 0; i < NK; ++i)
+                    kr[i] = __builtin_bit_cast(
+                        float4, __builtin_amdgcn_raw_buffer_load_b128(range, k_lane + i * k_step, 0, 0));
+            }
+        } else if (ok) {
+            const int rs = lane / LPR, c = (lane % LPR) * 4;
+#pragma unroll
+            for (int i = 0; i < NK; ++i) {
+                int key = key0 + 8 * wave + rs + RPI * i;
+                if (key > p.Tk - 1) key = p.Tk - 1;
+                const float* a = kb + key * p.k.st;
+                float t[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) t[j] = a[(c + j < p.d ? c + j : 0) * p.k.sd];
+                kr[i] = make_float4(t[0], t[1], t[2], t[3]);
+            }
+        }
+    }
+
+    __device__ __forceinline__ void store_k(char* ks, int wave, int lane) const {
+        const int rs = lane / LPR, i4 = lane % LPR;
+        const int c8 = i4 >> 1;            // 8-dim chunk 2t + h
+        char* base = ks + c8 * 512 + (i4 & 1) * 8;
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            const int r = 8 * wave + rs + RPI * i;
+            uint2 h, m, l;
+            split3(kr[i].x, kr[i].y, h.x, m.x, l.x);
+            split3(kr[i].z, kr[i].w, h.y, m.y, l.y);
+            char* a = base + ((r ^ (c8 & 15)) << 4);
+            *reinterpret_cast<uint2*>(a) = h;
+            *reinterpret_cast<uint2*>(a + K_PLANE) = m;
+            *reinterpret_cast<uint2*>(a + 2 * K_PLANE) = l;
+        }
+    }
+
+    // Wave w reads the 8 keys of (step s, lane half h) = (w / 2, w % 2).
+    __device__ __forceinline__ void load_v(const PrefillParams& p, const float* vb, int key0,
+                                           int wave, int lane, bool ok) {
+        if (VEC) {
+            const auto range = tile_range(vb, p.v.st, key0, p.Tk, p.d, ok);
+            if (ok && key0 + 32 <= p.Tk) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        vr[j][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            range, v_lane[j], v_row0 + (8 * (i >> 2) + (i & 3)) * v_st, 0));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        vr[j][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            range, v_lane[j] + v_row0 + (8 * (i >> 2) + (i & 3)) * v_st, 0, 0));
+            }
+        } else if (ok) {
+            const int k0 = key0 + 16 * (wave >> 1) + 4 * (wave & 1);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                int key = k0 + 8 * (i >> 2) + (i & 3);
+                if (key > p.Tk - 1) key = p.Tk - 1;
+                const float* a = vb + key * p.v.st;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const int dim = lane + 64 * j;
+                    vr[j][i] = a[(dim < p.d ? dim : 0) * p.v.sd];
+                }
+            }
+        }
+    }
+
+    __device__ __forceinline__ void store_v(char* vs, int wave, int lane) const {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int dim = lane + 64 * j;
+            if (64 * (j + 1) > D && dim >= D) continue;
+            uint4 h, m, l;
+            split3(vr[j][0], vr[j][1], h.x, m.x, l.x);
+            split3(vr[j][2], vr[j][3], h.y, m.y, l.y);
+            split3(vr[j][4], vr[j][5], h.z, m.z, l.z);
+            split3(vr[j][6], vr[j][7], h.w, m.w, l.w);
+            char* a = vs + (((dim >> 5) * 2 + (wave >> 1)) * 64 + (wave & 1) * 32 + (dim & 31)) * 16;
+            *reinterpret_cast<uint4*>(a) = h;
+            *reinterpret_cast<uint4*>(a + V_PLANE) = m;
+            *reinterpret_cast<uint4*>(a + 2 * V_PLANE) = l;
+        }
+    }
+};
+
+// One 32-row unit over key tiles [t0, t1) in plain f32 MFMAs on operands read
+// from global memory: the arithmetic for inputs outside the range in which the
+// three bf16 parts hold all 24 bits.  Slow, and rare.  Everything it needs is
+// derived here from a few opaque scalars, so that nothing of it is computed
+// ahead of, or kept in registers across, the main loop.
+template <int D, bool CAUSAL>
+__device__ __forceinline__ void unit_f32(const PrefillParams& p, int head, int unit, int t0, int t1,
+                                         floatx16 (&o)[D / 32], float& m_run, float& l_run) {
+    constexpr int NB = D / 32;
+    int tid = threadIdx.x;
+    float zero = 0.f;
+    asm volatile("" : "+v"(tid), "+v"(zero), "+s"(head), "+s"(unit), "+s"(t0), "+s"(t1));
+    const int l32 = tid & 31, half = (tid >> 5) & 1;
+    const int bi = head / p.Hkv, kvh = head % p.Hkv;
+    const int qrow = unit / p.G * 32 + l32;
+    const bool rok = qrow < p.Tq;
+    const float* qp = p.q.p + bi * p.q.sb + (kvh * p.G + unit % p.G) * p.q.sh + (int64_t)qrow * p.q.st;
+    const float* kb = p.k.p + bi * p.k.sb + kvh * p.k.sh;
+    const float* vb = p.v.p + bi * p.v.sb + kvh * p.v.sh;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[b][r] = zero;
+    m_run = kNegInf;
+    l_run = zero;
+#pragma nounroll
+    for (int kt = t0; kt < t1; ++kt) {
+        const int key0 = kt * 32;
+        const bool kok = key0 + l32 < p.Tk;
+        const float* kp = kb + (int64_t)(kok ? key0 + l32 : 0) * p.k.st;
+        floatx16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = zero;
+#pragma nounroll
+        for (int t = 0; t < D / 2; ++t) {
+            const int c = half * (D / 2) + t;
+            const float kx = kok && c < p.d ? kp[c * p.k.sd] : 0.f;
+            const float qx = rok && c < p.d ? qp[c * p.q.sd] * p.qscale : 0.f;
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kx, qx, s, 0, 0, 0);
+        }
+        float mt = kNegInf;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int key = key0 + 8 * (r >> 2) + 4 * half + (r & 3);
+            const bool vis = key < p.Tk && (!CAUSAL || key <= qrow + p.q_offset);
+            s[r] = vis ? s[r] : kNegInf;
+            mt = fmaxf(mt, s[r]);
+        }
+        const float m_new = fmaxf(m_run, pair_max(mt));
+        const float m_use = m_new == kNegInf ? 0.f : m_new;
+        const float alpha = fast_exp2(m_run - m_use);
+        l_run *= alpha;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+        m_run = m_new;
+        int key = key0 + 4 * half;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float pr = fast_exp2(s[r] - m_use);
+            l_run += pr;
+            asm volatile("" : "+v"(key));
+            const float* vp = vb + (int64_t)(key < p.Tk ? key : 0) * p.v.st;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const int dim = 32 * b + l32;
+                const float vx = key < p.Tk && dim < p.d ? vp[dim * p.v.sd] : 0.f;
+                o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx, pr, o[b], 0, 0, 0);
+            }
+            key += (r & 3) == 3 ? 5 : 1;
+            __builtin_amdgcn_sched_barrier(0);   // one key's V in registers at a time
+        }
+    }
+}
+
+// Two workgroups per CU for the persistent schedule, three up to 64 dims.  At
+// d = 128 the key-split variant (small problems, one short chunk per workgroup)
+// and the scalar-load variant (views that are not 16-byte vectors) take the
+// whole register file instead of spilling.
 template <int D, bool CAUSAL, bool VEC, bool SPLIT>
-__global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : 2) void prefill_mfma_kernel(const PrefillParams p) {
-    constexpr int KS = D + 4;          // K row stride in LDS (16-byte reads conflict-free)
-    constexpr int VS = D + 8;          // V row stride in LDS (lane halves on disjoint banks)
-    constexpr int STAGE = 32 * KS + 32 * VS;
+__global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : D <= 64 && !SPLIT ? 3 : 2) void prefill_mfma_kernel(const PrefillParams p) {
+    using Tile = SplitTile<D, VEC>;
     constexpr int NB = D / 32;         // 32-wide output column blocks
-    __shared__ __attribute__((aligned(16))) float lds[2 * STAGE];
+    constexpr int NT = D / 16;         // 16-dim steps of S^T
+    constexpr int KP = Tile::K_PLANE, VP = Tile::V_PLANE;
+    // At D = 128 the low parts of Q's last steps stay in LDS (16 registers that
+    // the two-wave budget of 256 does not hold).
+    constexpr int NQL = D == 128 && VEC && !SPLIT ? 4 : 0;
+    __shared__ __attribute__((aligned(16))) char lds[3 * (KP + VP) + NQL * 4096];
+    char* const Ks = lds;
+    char* const Vs = lds + 3 * KP;
+    char* const Qs = Vs + 3 * VP;
 
     // ---- persistent workgroup: slot q of XCD x -------------------------------
     // Hardware dispatches consecutive workgroup ids round-robin over the 8
@@ -197,7 +445,7 @@ __global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : 2) void pr
     // live across the whole persistent loop.
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const int bi = head / p.Hkv, kvh = head % p.Hkv;
 
@@ -227,27 +475,44 @@ __global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : 2) void pr
         t1 = min(n_tiles, t0 + p.chunk_tiles);
     }
 
-    // ---- Q^T fragment: qf[s] = Q[qrow][half*D/2 + s] * scale*log2(e) ----------
-    float qf[D / 2];
-    {
-        const float* qp = p.q.p + bi * p.q.sb + hq * p.q.sh + (int64_t)qrow * p.q.st;
-        const bool rok = active && qrow < p.Tq;
+    // ---- Q^T: three bf16 parts of Q[qrow][16t + 8*half + 0..7] * scale*log2(e)
+    short8 qf[2][NT], ql[NT - NQL];
+    char* const qls = Qs + (wave * NQL * 64 + lane) * 16;
+    const float* qp = p.q.p + bi * p.q.sb + hq * p.q.sh + (int64_t)qrow * p.q.st;
+    const bool rok = active && qrow < p.Tq;
+    uint32_t q_code = 0;
 #pragma unroll
-        for (int s4 = 0; s4 < D / 8; ++s4) {
-            const int c = half * (D / 2) + 4 * s4;
-            float x[4];
+    for (int t = 0; t < NT; ++t) {
+        const int c = 16 * t + 8 * half;
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
             if (VEC) {
-                float4 t = (rok && c < p.d) ? *reinterpret_cast<const float4*>(qp + c)
-                                            : make_float4(0.f, 0.f, 0.f, 0.f);
-                x[0] = t.x; x[1] = t.y; x[2] = t.z; x[3] = t.w;
+                const float4 t4 = (rok && c + j < p.d) ? *reinterpret_cast<const float4*>(qp + c + j)
+                                                       : make_float4(0.f, 0.f, 0.f, 0.f);
+                x[j] = t4.x; x[j + 1] = t4.y; x[j + 2] = t4.z; x[j + 3] = t4.w;
             } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) x[j] = (rok && c + j < p.d) ? qp[(c + j) * p.q.sd] : 0.f;
+                for (int u = 0; u < 4; ++u)
+                    x[j + u] = (rok && c + j + u < p.d) ? qp[(c + j + u) * p.q.sd] : 0.f;
             }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) qf[4 * s4 + j] = x[j] * p.qscale;
         }
+        uint4 h, m, l;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            x[j] *= p.qscale;
+            q_code = max(q_code, range_code(x[j]));
+        }
+        split3(x[0], x[1], h.x, m.x, l.x);
+        split3(x[2], x[3], h.y, m.y, l.y);
+        split3(x[4], x[5], h.z, m.z, l.z);
+        split3(x[6], x[7], h.w, m.w, l.w);
+        qf[0][t] = __builtin_bit_cast(short8, h);
+        qf[1][t] = __builtin_bit_cast(short8, m);
+        if (t < NT - NQL) ql[t < NT - NQL ? t : 0] = __builtin_bit_cast(short8, l);
+        else *reinterpret_cast<uint4*>(qls + (t - (NT - NQL)) * 1024) = l;
     }
+    asm volatile("" : "+v"(q_code));   // computed here, not from every x after the loop
 
     const float* kb = p.k.p + bi * p.k.sb + kvh * p.k.sh;
     const float* vb = p.v.p + bi * p.v.sb + kvh * p.v.sh;
@@ -270,10 +535,13 @@ __global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : 2) void pr
     const int kstep = rev ? -1 : 1;
     const int kfirst = rev ? t1 - 1 : t0;
     const int n_it = t1 - t0;
-    TileLoader<D, VEC> ld;
+    Tile ld;
+    ld.init(p, wave, lane);
     if (n_it > 0) {
-        ld.load(p, kb, vb, kfirst * 32, tid);
-        ld.store(lds, lds + 32 * KS, tid);
+        ld.load_k(p, kb, kfirst * 32, wave, lane, true);
+        ld.load_v(p, vb, kfirst * 32, wave, lane, true);
+        ld.store_k(Ks, wave, lane);
+        ld.store_v(Vs, wave, lane);
     }
     __syncthreads();
 
@@ -281,41 +549,59 @@ __global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : 2) void pr
         const int kt = kfirst + kstep * it;
         const bool has_next = it + 1 < n_it;
         const bool mine = kt < wave_tiles;
-        const float* Ks = lds + (it & 1) * STAGE;
-        const float* Vs = Ks + 32 * KS;
+        ld.load_k(p, kb, (kt + kstep) * 32, wave, lane, has_next);
         floatx16 s;
+        const float m_use = (m_run == kNegInf) ? 0.f : m_run;
         if (mine) {
-            // S^T = K Q^T  (32 keys x 32 rows), log2 domain.
+            // S^T - m = K Q^T - m  (32 keys x 32 rows), log2 domain: first every
+            // small product, then the products of the high parts, so that only
+            // D/16 sums are rounded at the size of the score.
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = 0.f;
-            const float* krow = Ks + l32 * KS + half * (D / 2);
+            for (int r = 0; r < 16; ++r) s[r] = -m_use;
+            const int kbase = half * 512 + ((l32 ^ half) << 4);
             // Raised issue priority while this wave feeds the MFMA pipe, so the
             // two waves sharing a SIMD alternate MFMA and softmax phases.
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int t = 0; t < D / 8; ++t) {
-                const float4 kq = *reinterpret_cast<const float4*>(krow + 4 * t);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.x, qf[4 * t + 0], s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.y, qf[4 * t + 1], s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.z, qf[4 * t + 2], s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.w, qf[4 * t + 3], s, 0, 0, 0);
+            for (int t = 0; t < NT; ++t) {
+                const char* a = Ks + t * 1024 + (kbase ^ ((2 * t & 15) << 4));
+                const short8 kh = *reinterpret_cast<const short8*>(a);
+                const short8 km = *reinterpret_cast<const short8*>(a + KP);
+                const short8 kl = *reinterpret_cast<const short8*>(a + 2 * KP);
+                s = mfma_bf16(kl, qf[0][t], s);
+                s = mfma_bf16(kh, t < NT - NQL ? ql[t < NT - NQL ? t : 0]
+                                               : *reinterpret_cast<const short8*>(
+                                                     qls + (t - (NT - NQL)) * 1024), s);
+                s = mfma_bf16(km, qf[1][t], s);
+                s = mfma_bf16(km, qf[0][t], s);
+                s = mfma_bf16(kh, qf[1][t], s);
             }
-            // Schedule: the first 4 K reads, then one read per 4 MFMAs, so
-            // reads run 4 chunks (16 MFMAs) ahead of their use.
 #pragma unroll
-            for (int i = 0; i < 4; ++i) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            for (int t = 0; t < NT; ++t) {
+                const char* a = Ks + t * 1024 + (kbase ^ ((2 * t & 15) << 4));
+                s = mfma_bf16(*reinterpret_cast<const short8*>(a), qf[0][t], s);
+            }
+            // Schedule: the operands of a step are read one step ahead.
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
 #pragma unroll
-            for (int i = 0; i < D / 8 - 4; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            for (int t = 0; t < NT - 1; ++t) {
+                if (t + 1 < NT - NQL) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                else __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 5, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 5, 0);
+#pragma unroll
+            for (int t = 0; t < NT - 2; ++t) {
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
-
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
             __builtin_amdgcn_s_setprio(0);
         }
-        // The next tile's loads are issued after the QK^T MFMAs, so their
-        // registers and the K operands are never live at the same time.
-        if (has_next) ld.load(p, kb, vb, (kt + kstep) * 32, tid);
+        __syncthreads();   // every wave has read K; V is visible
+        if (has_next) ld.store_k(Ks, wave, lane);
+        ld.load_v(p, vb, (kt + kstep) * 32, wave, lane, has_next);
         if (mine) {
             // Mask keys past T_k and (causal) keys after row + q_offset.
             const int key0 = kt * 32;
@@ -338,54 +624,74 @@ __global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : 2) void pr
 #pragma unroll
             for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
             mt = pair_max(mt);
-            if (__builtin_amdgcn_ballot_w64(mt > m_run + 8.f) != 0) {
-                const float m_new = fmaxf(m_run, mt);
-                const float alpha = fast_exp2(m_run - ((m_new == kNegInf) ? 0.f : m_new));
+            if (__builtin_amdgcn_ballot_w64(mt > (m_run == kNegInf ? kNegInf : 8.f)) != 0) {
+                const float m_new = fmaxf(m_run, mt + m_use);
+                const float n_use = (m_new == kNegInf) ? 0.f : m_new;
+                const float alpha = fast_exp2(m_run - n_use);
                 l_run *= alpha;
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] -= n_use - m_use;
                 m_run = m_new;
             }
-            const float m_use = (m_run == kNegInf) ? 0.f : m_run;
             float ls = 0.f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                s[r] = fast_exp2(s[r] - m_use);
+                s[r] = fast_exp2(s[r]);
                 ls += s[r];
             }
             l_run += ls;
 
-            // O^T += V^T P^T ; reduction step r pairs key 8*(r/4)+4*half+r%4.
+            // O^T += V^T P^T ; step st takes the keys of registers 8st .. 8st+7.
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float* vrow = Vs + (8 * (r >> 2) + 4 * half + (r & 3)) * VS + l32;
+            for (int st = 0; st < 2; ++st) {
+                uint4 h, m, l;
+                split3(s[8 * st + 0], s[8 * st + 1], h.x, m.x, l.x);
+                split3(s[8 * st + 2], s[8 * st + 3], h.y, m.y, l.y);
+                split3(s[8 * st + 4], s[8 * st + 5], h.z, m.z, l.z);
+                split3(s[8 * st + 6], s[8 * st + 7], h.w, m.w, l.w);
+                const short8 ph = __builtin_bit_cast(short8, h), pm = __builtin_bit_cast(short8, m),
+                             pl = __builtin_bit_cast(short8, l);
 #pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * b], s[r], o[b], 0, 0, 0);
+                for (int b = 0; b < NB; ++b) {
+                    const char* a = Vs + ((b * 2 + st) * 64 + lane) * 16;
+                    const short8 vh = *reinterpret_cast<const short8*>(a);
+                    const short8 vm = *reinterpret_cast<const short8*>(a + VP);
+                    const short8 vl = *reinterpret_cast<const short8*>(a + 2 * VP);
+                    o[b] = mfma_bf16(vl, ph, o[b]);
+                    o[b] = mfma_bf16(vh, pl, o[b]);
+                    o[b] = mfma_bf16(vm, pm, o[b]);
+                    o[b] = mfma_bf16(vm, ph, o[b]);
+                    o[b] = mfma_bf16(vh, pm, o[b]);
+                    o[b] = mfma_bf16(vh, ph, o[b]);
+                }
             }
-            // Schedule: V operands are read (two per ds_read2) 4 reads ahead of
-            // the MFMAs that use them.
-            constexpr int NVR = 16 * NB / 2;       // ds_read2_b32 per tile
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-#pragma unroll
-            for (int i = 0; i < NVR - 4; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            for (int i = 0; i < 2 * NB - 1; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
             __builtin_amdgcn_s_setprio(0);
         }
-
-        if (has_next) {
-            float* ks = lds + ((it + 1) & 1) * STAGE;
-            ld.store(ks, ks + 32 * KS, tid);
-        }
-        __syncthreads();
+        __syncthreads();   // every wave has read V; the next K is visible
+        if (has_next) ld.store_v(Vs, wave, lane);
     }
+
+    // Inputs the bf16 parts do not hold show in the result; such a unit is
+    // computed again in f32.
+    uint32_t o_code = 0;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_code = max(o_code, range_code(o[b][r]));
+    if (__builtin_amdgcn_ballot_w64(q_code > kQueryCodes || o_code >= kResultCodes) != 0)
+        unit_f32<D, CAUSAL>(p, head, unit, t0, min(t1, wave_tiles), o, m_run, l_run);
 
     float l_tot = pair_sum(l_run);
     if constexpr (SPLIT) {
@@ -432,19 +738,18 @@ __global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : 2) void pr
 #pragma unroll
                 for (int u = 0; u < GRP; ++u) {
                     // A missing last record of a group reads this chunk's own
-                    // (finite) record with weight exp2(-inf) = 0.
-                    const bool ok = i + u < n_parts;
-                    const int64_t sl = ((int64_t)(slot0 + (ok ? i + u : chunk)) * 4 + wave);
+                    // record again and is not combined.
+                    const int64_t sl = ((int64_t)(slot0 + (i + u < n_parts ? i + u : chunk)) * 4 + wave);
                     const float* ro = p.ws + o_base + sl * (D / 2) * 64 + lane;
                     const float* rml = p.ws + (sl * 64 + lane) * 2;
-                    const float m_ld = load_coherent(rml), l_ld = load_coherent(rml + 1);
-                    mc[u] = ok ? m_ld : kNegInf;
-                    lc[u] = ok ? l_ld : 0.f;
+                    mc[u] = load_coherent(rml);
+                    lc[u] = load_coherent(rml + 1);
 #pragma unroll
                     for (int e = 0; e < D / 2; ++e) oc[u][e] = load_coherent(ro + e * 64);
                 }
 #pragma unroll
                 for (int u = 0; u < GRP; ++u) {
+                    if (i + u >= n_parts) break;
                     const float m_new = fmaxf(M, mc[u]);
                     const float mu = m_new == kNegInf ? 0.f : m_new;
                     const float a = fast_exp2(M - mu), bw = fast_exp2(mc[u] - mu);
@@ -921,6 +1226,9 @@ hipError_t launch_prefill_wide(PrefillParams p, bool causal, hipStream_t stream)
 hipError_t launch_prefill(PrefillParams p, bool causal, bool vec, hipStream_t stream) {
     derive_schedule(p);
     if (p.total == 0) return hipSuccess;
+    // The vector loads of a K/V tile hold its row offsets in 32 bits.
+    constexpr int64_t kMaxRowStride = 1 << 24;
+    vec = vec && p.k.st >= 0 && p.k.st < kMaxRowStride && p.v.st >= 0 && p.v.st < kMaxRowStride;
     switch (prefill_padded_dim(p.d)) {
         case 32: return launch_d<32>(p, causal, vec, stream);
         case 64: return launch_d<64>(p, causal, vec, stream);

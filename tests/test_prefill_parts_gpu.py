@@ -1,0 +1,107 @@
+"""Prefill on the bf16 matrix cores: f32 operands as three bf16 parts.
+
+The results against 64 bits (at most 4e-6 of the result's norm: a few f32
+roundings of sums of d products and of up to T_k weights), at the edges of the
+32-key and 32-row tiles and of the 16-dim steps, and for values the parts do
+not hold (infinities, magnitudes near both ends of f32), which a unit computes
+again in f32.
+"""
+import numpy as np
+import pytest
+import torch
+
+import nne_testlib as T
+
+pytestmark = pytest.mark.gpu
+
+
+def attend64(q, k, v, causal, offset=0):
+    g = q.shape[1] // k.shape[1]
+    k, v = (np.repeat(x.astype(np.float64), g, 1) for x in (k, v))
+    s = np.einsum("bhqd,bhkd->bhqk", q.astype(np.float64), k) / np.sqrt(q.shape[3])
+    if causal:
+        s = np.where(np.arange(s.shape[3]) > np.arange(s.shape[2])[:, None] + offset, -np.inf, s)
+    w = np.exp(s - s.max(-1, keepdims=True))
+    return np.einsum("bhqk,bhkd->bhqd", w / w.sum(-1, keepdims=True), v)
+
+
+def run(q, k, v, causal, offset=0):
+    nne = T.load_package()
+    dev = [torch.from_numpy(x).cuda() for x in (q, k, v)]
+    o = nne.attention_forward(*dev, causal, q_offset=offset)
+    torch.cuda.synchronize()
+    return o.cpu().numpy()
+
+
+def draw(seed, b, hq, hkv, tq, tk, d):
+    rng = np.random.default_rng(seed)
+    return (rng.standard_normal((b, h, t, d)).astype(np.float32)
+            for h, t in ((hq, tq), (hkv, tk), (hkv, tk)))
+
+
+def check64(o, ref):
+    assert np.isfinite(o).all()
+    assert np.linalg.norm(o - ref) <= 4e-6 * np.linalg.norm(ref)
+
+
+# Enough heads for the unsplit launch, then few enough for the key split.
+@pytest.mark.parametrize("heads", [(40, 20), (2, 1)])
+@pytest.mark.parametrize("d", [4, 20, 32, 36, 64, 68, 100, 128])
+@pytest.mark.parametrize("tq,tk,causal", [(97, 289, False), (289, 289, True), (320, 1, False),
+                                          (33, 320, True), (300, 31, False)])
+def test_tile_edges(heads, d, tq, tk, causal):
+    q, k, v = draw(d + tq, 2, heads[0], heads[1], tq, tk, d)
+    check64(run(q, k, v, causal, tk - tq), attend64(q, k, v, causal, tk - tq))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("qs,ks,vs", [(1.0, 1.0, 1e-37), (1.0, 1.0, 1e34), (1e-30, 1e30, 1.0),
+                                      (1e30, 1e-30, 1.0), (1e-36, 1e36, 1e-36)])
+def test_magnitudes_near_the_ends_of_f32(d, qs, ks, vs):
+    q, k, v = draw(7, 2, 40, 20, 300, 300, d)
+    q, k, v = q * np.float32(qs), k * np.float32(ks), v * np.float32(vs)
+    ref = attend64(q, k, v, True)
+    scale = 1 / np.abs(ref).max()      # norms of 1e34-sized values leave f32
+    check64(run(q, k, v, True).astype(np.float64) * scale, ref * scale)
+
+
+# One batch element takes the key split, four the unsplit launch.
+@pytest.mark.parametrize("b", [1, 4])
+@pytest.mark.parametrize("d", [64, 128])
+def test_keys_of_minus_infinity_have_no_weight(b, d):
+    q, k, v = draw(8, b, 40, 20, 300, 300, d)
+    q = np.abs(q) + np.float32(0.01)      # q . k = -inf for every row
+    k[:, 3, 250] = -np.inf
+    k[:, 7, 5] = -np.inf
+    check64(run(q, k, v, False), attend64(q, np.maximum(k, np.float32(-1e30)), v, False))
+
+
+@pytest.mark.parametrize("b", [1, 4])
+@pytest.mark.parametrize("d", [64, 128])
+def test_nan_and_infinity_reach_the_rows_that_see_them(b, d):
+    q, k, v = draw(9, b, 40, 20, 300, 300, d)
+    ref = attend64(q, k, v, True)
+    v[0, 2, 200, 3] = np.inf
+    k[0, 4, 100, 0] = np.nan
+    o = run(q, k, v, True)
+    assert np.isposinf(o[0, 4:6, 200:, 3]).all()
+    assert np.isnan(o[0, 8:10, 100:]).all()
+    # Rows of earlier key tiles, and every other head, are as without them.
+    check64(o[0, 4:6, :192], ref[0, 4:6, :192])
+    check64(o[0, 8:10, :96], ref[0, 8:10, :96])
+    others = [h for h in range(40) if h not in (4, 5, 8, 9)]
+    check64(o[:, others], ref[:, others])
+
+
+def test_row_strides_beyond_the_vector_loads():
+    """K/V rows 2^24 floats apart take the scalar-load variant."""
+    tk, d, st = 40, 64, 1 << 24
+    q, k, v = draw(10, 1, 2, 1, 64, tk, d)
+    big = torch.empty(tk * st, device="cuda")
+    kd, vd = (torch.as_strided(big, (1, 1, tk, d), (tk * st, tk * st, st, 1), off) for off in (0, 512))
+    kd.copy_(torch.from_numpy(k))
+    vd.copy_(torch.from_numpy(v))
+    nne = T.load_package()
+    o = nne.attention_forward(torch.from_numpy(q).cuda(), kd, vd, False)
+    torch.cuda.synchronize()
+    check64(o.cpu().numpy(), attend64(q, k, v, False))
