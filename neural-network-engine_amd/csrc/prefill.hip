@@ -386,19 +386,18 @@ __device__ __forceinline__ void unit_f32(const PrefillParams& p, int head, int u
     }
 }
 
-// Two workgroups per CU for the persistent schedule, three up to 64 dims.  At
-// d = 128 the key-split variant (small problems, one short chunk per workgroup)
-// and the scalar-load variant (views that are not 16-byte vectors) take the
+// Two workgroups per CU, three up to 64 dims for the persistent schedule.  At
+// d = 128 the scalar-load variant (views that are not 16-byte vectors) takes the
 // whole register file instead of spilling.
 template <int D, bool CAUSAL, bool VEC, bool SPLIT>
-__global__ __launch_bounds__(256, (D >= 128 && (SPLIT || !VEC)) ? 1 : D <= 64 && !SPLIT ? 3 : 2) void prefill_mfma_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 : 2) void prefill_mfma_kernel(const PrefillParams p) {
     using Tile = SplitTile<D, VEC>;
     constexpr int NB = D / 32;         // 32-wide output column blocks
     constexpr int NT = D / 16;         // 16-dim steps of S^T
     constexpr int KP = Tile::K_PLANE, VP = Tile::V_PLANE;
     // At D = 128 the low parts of Q's last steps stay in LDS (16 registers that
     // the two-wave budget of 256 does not hold).
-    constexpr int NQL = D == 128 && VEC && !SPLIT ? 4 : 0;
+    constexpr int NQL = D == 128 && VEC ? 4 : 0;
     __shared__ __attribute__((aligned(16))) char lds[3 * (KP + VP) + NQL * 4096];
     char* const Ks = lds;
     char* const Vs = lds + 3 * KP;
@@ -1188,19 +1187,28 @@ PrefillSplit prefill_split_plan(PrefillParams& p, bool causal, bool vec) {
         max_t = std::max(max_t, tiles[w]);
     }
     if (max_t < 4) return r;
-    // One workgroup per CU: measured against two per CU where they fit (d = 64),
-    // the longer chunks with half the records and prologues are faster
-    // (GPT-2 prompt, T = 1024: 33.9 against 31.0 us).
-    const int64_t slots = cus;
-    // Smallest chunk (<= 16 chunks per item) whose non-empty chunks fill the
-    // CUs at most once.  One-tile chunks, where they fit, beat two-tile ones
-    // (config 1: 12.4 against 13.0 us): the chain of tiles halves, the merge
-    // grows by one round trip.
-    int ch = std::max(1, (max_t + 15) / 16);
-    for (;; ++ch) {
-        int64_t n = 0;
-        for (int w = 0; w < p.n_wg; ++w) n += std::max(1, (tiles[w] + ch - 1) / ch);
-        if (n * p.B * p.Hkv <= slots || ch >= max_t) break;
+    // One or two workgroups per CU (k), and for each the smallest chunk (at most
+    // 16 chunks per item) whose chunks fit.  Two share the CU's matrix cores but
+    // fill each other's waits; more parts cost the last chunk more records.
+    // Fitted to measured calls (us, k = 1 / k = 2, chunk tiles and parts in
+    // brackets): d = 128, 333 rows over 3001 keys 153 [47, 2] / 108 [19, 5], T =
+    // 2610 72 [17, 5] / 66 [8, 11], T = 509 GQA 36 [6, 3] / 39 [3, 6], T = 512
+    // non-causal 30 [4, 4] / 39 [2, 8]; d = 64, T = 3517 61 [28, 4] / 52 [13, 9],
+    // T = 448 19 [4, 4] / 20 [2, 7].  Three per CU were slower than two throughout.
+    const double tile_us[2] = {D == 128 ? 3.1 : 1.7, D == 128 ? 4.6 : 2.4};
+    const double start_us[2] = {D == 128 ? 14.0 : 9.0, D == 128 ? 18.0 : 10.0};
+    const double part_us = D == 128 ? 1.3 : 1.0;
+    int ch = 0;
+    double best = 1e300;
+    for (int k = 1; k <= (D > 32 ? 2 : 1); ++k) {
+        int c = std::max(1, (max_t + 15) / 16);
+        for (;; ++c) {
+            int64_t n = 0;
+            for (int w = 0; w < p.n_wg; ++w) n += std::max(1, (tiles[w] + c - 1) / c);
+            if (n * p.B * p.Hkv <= (int64_t)k * cus || c >= max_t) break;
+        }
+        const double us = tile_us[k - 1] * c + start_us[k - 1] + part_us * ((max_t + c - 1) / c);
+        if (us < best) { best = us; ch = c; }
     }
     const int nc = (max_t + ch - 1) / ch;
     if (nc < 2) return r;
