@@ -121,11 +121,15 @@ int nne_counters_init(uint32_t *counters, uint64_t n, void *stream);
  * (:113).  Rows that see no key are zero (:186-194).  `o` has Q's shape.
  * Any head dim; above 128 the tensors must be 16-byte vector views
  * (d % 4 == 0, unit dim stride, other strides multiples of 4, 16-byte
- * aligned) -- NNE_EINVAL otherwise.  Above 256 dims a separate kernel runs
- * (MFMA, K/V read straight into operand layout), and so do 129-255 dims and
- * d = 256 problems too small to fill the device on the 256-dim kernel;
- * problems with too few query rows to fill the device split their keys over
- * several workgroups, with records in the workspace. */
+ * aligned) -- NNE_EINVAL otherwise.  Above 128 dims problems with more 32-row
+ * units than the device has CUs (causal above 256 dims: than two per CU) run on
+ * an 8-wave kernel up to 512 dims; all others on a kernel for any head dim
+ * (K/V read straight into MFMA operand layout), where problems with too few
+ * query rows to fill the device split their keys over several workgroups, with
+ * records in the workspace.
+ * Products are those of f32 operands: each operand is the exact sum of three
+ * bf16 parts on the bf16 matrix cores, or taken whole on the f32 ones, and all
+ * sums are f32. */
 int nne_flash_attention_forward(const float *q, const int64_t q_shape[4], const int64_t q_strides[4],
                                 const float *k, const int64_t k_shape[4], const int64_t k_strides[4],
                                 const float *v, const int64_t v_shape[4], const int64_t v_strides[4],

@@ -223,19 +223,21 @@ int deep_workspace(nne::DeepParams& p, int max_tiles, const nne_workspace_t* wsp
     return NNE_OK;
 }
 
-// Head dims 129-256 with more query rows per KV head than the split-K kernel
-// takes: the wave-pair kernel at d = 256 when its work items (4 units of 32
-// rows each) fill the device, else the deep kernel's 2-wave form, which pads
-// no dims to 256 and spreads (or key-splits) small problems over the CUs.
-// (Measured: d = 192 B = 8, H = 20, T = 1500 3.32 -> 2.56 ms; d = 256 causal
-// B = 1, H = 8, T = 1024 0.28 -> 0.17 ms; at d = 256 with the device full the
-// wave-pair kernel is level or up to 2 % faster.)
-bool wide_on_deep(int64_t B, int64_t Hkv, int64_t G, int64_t Tq, int d) {
-    if (nne::prefill_padded_dim(d) != 0 || nne::splitk_padded_dim(d) == 0) return false;
-    if (G * Tq <= nne::splitk_max_rows()) return false;
-    if (d != 256) return true;
-    const int64_t items = B * Hkv * ((G * ((Tq + 31) / 32) + 3) / 4);
-    return items < device_cus();
+// Head dims 129-512 with more query rows per KV head than the split-K kernel
+// takes: the 8-wave kernel when there are more 32-row units than CUs (above
+// 256 dims, causal: than two per CU, whose lengths then even out), else the
+// deep kernel, which spreads or key-splits them over every CU.  Measured on
+// both sides (deep / 8-wave, us): d = 256, T = 1024, 8 heads (256 units) 164 /
+// 163 and 10 heads 273 / 173; T = 64, 128 heads (256 units) 18 / 20; d = 512
+// non-causal, T = 512, 16 heads (256 units) 88 / 120, T = 1024, 10 heads (320)
+// 292 / 227; causal, T = 1024, 16 heads (512 units) 178 / 228, 20 heads (640)
+// 323 / 296, T = 4096, 16 heads 2414 / 2007.
+bool on_deep(int64_t B, int64_t Hkv, int64_t G, int64_t Tq, int d, bool causal) {
+    if (nne::prefill_padded_dim(d) != 0) return false;
+    if (d > 512) return true;
+    if (G * Tq <= nne::splitk_max_rows()) return nne::splitk_padded_dim(d) == 0;
+    const int64_t units = B * Hkv * G * ((Tq + 31) / 32);
+    return units <= (int64_t)device_cus() * (d > 256 && causal ? 2 : 1);
 }
 
 // Records of the largest key split a deep-kernel problem of these shapes
@@ -264,15 +266,18 @@ int run_attention(const float* q, const int64_t* qs_, const int64_t* qst, const 
     const int B = (int)qs_[0], Hq = (int)qs_[1], Tq = (int)qs_[2], d = (int)qs_[3];
     const int Hkv = (int)ks_[1], Tk = (int)ks_[2];
     if ((int64_t)B * Hq * Tq == 0 || d == 0) return NNE_OK;
-    // Head dims above 128 (d <= 256) run on the wave-pair MFMA kernel or the
-    // deep kernel's 2-wave form (wide_on_deep), or on the split-K kernel when a
-    // KV head has few query rows; above 256 on the deep kernel.
+    // Head dims above 128 run on the 8-wave MFMA kernel or the deep kernel
+    // (on_deep), or up to 256 dims on the split-K kernel when a KV head has few
+    // query rows.
     const bool wide = nne::prefill_padded_dim(d) == 0;
-    // (At 129-256 dims K/V row strides outside the deep kernel's 32-bit tile
-    // offsets keep the wave-pair kernel.)
+    // K/V row strides outside the deep kernel's 32-bit tile offsets keep the
+    // 8-wave kernel up to 256 dims; strides outside that kernel's vector loads
+    // keep the deep kernel above.
     const bool deep_strides = kst[2] >= 0 && vst[2] >= 0 && kst[2] < (1 << 25) && vst[2] < (1 << 25);
-    const bool deep = wide && (nne::splitk_padded_dim(d) == 0 ||
-                               (deep_strides && wide_on_deep(B, Hkv, Hq / Hkv, Tq, d)));
+    const bool wide_strides = kst[2] >= 0 && vst[2] >= 0 && kst[2] < nne::kMaxTileStride &&
+                              vst[2] < nne::kMaxTileStride;
+    const bool deep = wide && (d > 256 ? !wide_strides || on_deep(B, Hkv, Hq / Hkv, Tq, d, causal)
+                                       : deep_strides && on_deep(B, Hkv, Hq / Hkv, Tq, d, causal));
     // Offsets beyond +-2^30 cannot change visibility for int32 lengths.
     const int qoff = (int)std::max<int64_t>(-(1 << 30), std::min<int64_t>(q_offset, 1 << 30));
     const bool vec = d % 4 == 0 && vec_view(q, qst) && vec_view(k, kst) && vec_view(v, vst) &&
@@ -420,7 +425,7 @@ nne_workspace_size_t attention_workspace(const int64_t* qs_, const int64_t* ks_,
     const int qoff = (int)std::max<int64_t>(-(1 << 30), std::min<int64_t>(q_offset, 1 << 30));
     // The deep kernel's key split: above 256 dims, and head dims 129-256 on its
     // 2-wave form.
-    if (nne::splitk_padded_dim(d) == 0 || (Hq % Hkv == 0 && wide_on_deep(B, Hkv, Hq / Hkv, Tq, d))) {
+    if (nne::splitk_padded_dim(d) == 0 || (Hq % Hkv == 0 && on_deep(B, Hkv, Hq / Hkv, Tq, d, causal))) {
         if (d % 4 == 0 && Hq % Hkv == 0)
             r.records_bytes = deep_workspace_bytes(B, Hq, Hkv, Tq, d, deep_max_tiles(Tk, causal, qoff, Tq));
         return r;
@@ -428,7 +433,7 @@ nne_workspace_size_t attention_workspace(const int64_t* qs_, const int64_t* ks_,
     const bool wide = nne::prefill_padded_dim(d) == 0;
     const int64_t rows = (int64_t)(Hq / Hkv) * Tq;
     const int64_t tk = causal ? std::min<int64_t>(Tk, (int64_t)qoff + Tq) : Tk;
-    // Wide head dims with more rows per KV head take the wave-pair kernel,
+    // Wide head dims with more rows per KV head take the 8-wave kernel,
     // which needs no workspace.
     const bool wide_mfma = wide && rows > nne::splitk_max_rows();
     if (d % 4 == 0 && !wide_mfma && (wide || (rows <= nne::splitk_max_rows() && tk > 0))) {

@@ -21,7 +21,8 @@ int splitk_rows_per_launch(int d);
 // `vec` selects 16-byte loads/stores: requires dim stride 1, d % 4 == 0,
 // 16-byte aligned base pointers and row/head/batch strides that are multiples of 4.
 hipError_t launch_prefill(PrefillParams p, bool causal, bool vec, hipStream_t stream);
-// Head dims 129..256 (16-byte vector views): the wave-pair MFMA kernel.
+// Head dims 129..512 (16-byte vector views; above 256 K/V row strides in
+// [0, kMaxTileStride)): the 8-wave MFMA kernel.
 hipError_t launch_prefill_wide(PrefillParams p, bool causal, hipStream_t stream);
 // Head dims above 256 (deep.hip; d % 4 == 0, 16-byte vector views of Q, K,
 // V and O): prefill, cross-attention and decode over a KV cache (p.lens).

@@ -33,6 +33,7 @@ struct OutView4 {
 // 4w .. 4w+3, so the G query heads of a group share every K/V tile the
 // workgroup stages in LDS.
 constexpr int kMaxSplitItems = 256;   // work items per KV head of a key-split launch
+constexpr int64_t kMaxTileStride = 1 << 24;   // K/V row strides (floats) below this, from 0, are read as vectors
 
 struct PrefillParams {
     View4 q, k, v;
@@ -75,7 +76,7 @@ struct PrefillParams {
 };
 
 // Head dims above 256 (deep.hip), prefill, cross-attention and decode alike,
-// and prefill at 129-256 dims the wave-pair kernel does not take.  The G * Tq
+// and prefill at 129-512 dims the 8-wave kernel does not take.  The G * Tq
 // query rows of a KV head are flattened (row r: query head kvh * G + r / Tq,
 // position r % Tq) and cut into 32-row units; a workgroup serves one unit and
 // one kDeepChunk-dim chunk of the output dims (256 dims on the 2-wave form,

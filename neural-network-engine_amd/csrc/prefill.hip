@@ -7,7 +7,7 @@
 // skipped (:101-104) -- generalised to grouped-query heads (KV head hq / G) and
 // a causal offset.
 //
-// MI355X mapping (head dims up to 128; 129-256 dims: prefill_wide_kernel).
+// MI355X mapping (head dims up to 128; 129-512 dims: prefill_wide_kernel).
 // Every f32 operand is the exact sum of three bf16 parts and every product the
 // six largest products of parts (nne_common.hpp), on v_mfma_f32_32x32x16_bf16.
 // One wave owns 32 query rows and computes the score tile transposed,
@@ -61,53 +61,6 @@ namespace nne {
 
 namespace {
 
-template <int D, bool VEC, int THREADS = 256>
-struct TileLoader {
-    // K/V tile of 32 keys x D dims = 8*D float4; 256 threads -> D/32 each.
-    static constexpr int NV = 8 * D / THREADS;
-    static constexpr int C4 = D / 4;    // float4 columns per row
-    static_assert(NV * THREADS == 8 * D, "whole tile per pass");
-    float4 kr[NV], vr[NV];
-
-    __device__ __forceinline__ void load(const PrefillParams& p, const float* kb, const float* vb,
-                                         int key0, int tid) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int idx = tid + THREADS * i;
-            const int row = idx / C4, c = (idx % C4) * 4;
-            const int key = key0 + row;
-            if (VEC) {
-                const bool ok = key < p.Tk && c < p.d;
-                kr[i] = ok ? *reinterpret_cast<const float4*>(kb + key * p.k.st + c)
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
-                vr[i] = ok ? *reinterpret_cast<const float4*>(vb + key * p.v.st + c)
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
-            } else {
-                float kx[4], vx[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const bool ok = key < p.Tk && c + j < p.d;
-                    kx[j] = ok ? kb[key * p.k.st + (c + j) * p.k.sd] : 0.f;
-                    vx[j] = ok ? vb[key * p.v.st + (c + j) * p.v.sd] : 0.f;
-                }
-                kr[i] = make_float4(kx[0], kx[1], kx[2], kx[3]);
-                vr[i] = make_float4(vx[0], vx[1], vx[2], vx[3]);
-            }
-        }
-    }
-
-    __device__ __forceinline__ void store(float* ks, float* vs, int tid) const {
-        constexpr int KS = D + 4, VS = D + 8;
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int idx = tid + THREADS * i;
-            const int row = idx / C4, c = (idx % C4) * 4;
-            *reinterpret_cast<float4*>(ks + row * KS + c) = kr[i];
-            *reinterpret_cast<float4*>(vs + row * VS + c) = vr[i];
-        }
-    }
-};
-
 // Last key index visible to any row of row block rb (or -1).
 __device__ __forceinline__ int last_visible_key(const PrefillParams& p, int rb, bool causal) {
     if (!causal) return p.Tk - 1;
@@ -158,7 +111,7 @@ __device__ __forceinline__ int item_at(const PrefillParams& p, int j, int x, int
     return 1;
 }
 
-// K/V tile of 32 keys x D dims, read by 256 threads and left in LDS as three
+// K/V tile of 32 keys x D dims, read by 4 or 8 waves and left in LDS as three
 // bf16 planes each, in operand order (one 16-byte slot per lane):
 //   K (A of S^T = K Q^T): plane p, 16-dim step t, lane half h, key r at slot
 //     (p * D/16 + t) * 64 + h * 32 + (r ^ ((2t + h) & 15)), dims 16t + 8h .. + 7.
@@ -171,30 +124,49 @@ __device__ __forceinline__ int item_at(const PrefillParams& p, int j, int x, int
 // Rows past T_k are zeros, or with scalar loads row T_k - 1 again (their
 // weights are zero); dims past d read dim 0 (Q is zero there, and those output
 // dims are not stored).
-template <int D, bool VEC>
+template <int D, bool VEC, int WAVES = 4>
 struct SplitTile {
     static constexpr int NB = D / 32;
     static constexpr int K_PLANE = 32 * D * 2, V_PLANE = 32 * D * 2;   // bytes
-    static constexpr int LPR = D / 4;                // lanes per key row (4 dims each)
-    static constexpr int RPI = 64 / LPR;             // rows per load
-    static constexpr int NK = 8 / RPI;               // K loads per thread
-    static_assert(64 % LPR == 0 && 8 % RPI == 0, "whole rows per load");
-    static constexpr int NJ = (D + 63) / 64;         // dims per lane of V
+    static constexpr int LPR = D / 4;                      // lanes per key row (4 dims each)
+    static constexpr int NC = (LPR + 63) / 64;            // loads per key row
+    static constexpr int RPI = LPR <= 64 ? 64 / LPR : 1;   // rows per load
+    static constexpr int KR = 32 / WAVES;                  // key rows per wave
+    static constexpr int NK = KR / RPI * NC;               // K loads per thread
+    static constexpr int VD = D / (WAVES / 4);             // dims per wave of V
+    static constexpr int NJ = (VD + 63) / 64;              // dims per lane of V
+    static_assert(KR % RPI == 0 && LPR <= 64 * NC, "whole rows per load");
     float4 kr[NK];
     float vr[NJ][8];
     // VEC views (row strides in [0, 2^24)): byte offsets of this lane within a
     // tile and of each load's rows, so that a tile's loads need only its base.
-    uint32_t k_lane, k_step, v_lane[NJ], v_row0, v_st;
+    uint32_t k_lane[NC], k_step, v_lane[NJ], v_row0, v_st;
+
+    // This lane's row among a load's and its first dim in load column j (a row
+    // of 96 dims leaves the lanes past two rows to repeat the second).
+    static __device__ __forceinline__ int row_of(int lane) { return min(lane / LPR, RPI - 1); }
+    static __device__ __forceinline__ int col_of(int lane, int j) {
+        return NC > 1 ? min((lane + 64 * j) * 4, D - 4) : lane < LPR * RPI ? (lane % LPR) * 4 : D - 4;
+    }
+    static __device__ __forceinline__ int dim_of(int wave, int lane, int j) {
+        return (wave >> 2) * VD + lane + 64 * j;
+    }
 
     __device__ __forceinline__ void init(const PrefillParams& p, int wave, int lane) {
-        const int c = (lane % LPR) * 4;
         const uint32_t kst = (uint32_t)p.k.st * 4u, vst = (uint32_t)p.v.st * 4u;
-        k_lane = (8 * wave + lane / LPR) * kst + (c < p.d ? c : 0) * 4;
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int c = col_of(lane, j);
+            k_lane[j] = (KR * wave + row_of(lane)) * kst + (c < p.d ? c : 0) * 4;
+        }
         k_step = RPI * kst;
-        v_row0 = (16 * (wave >> 1) + 4 * (wave & 1)) * vst;
+        v_row0 = (16 * ((wave >> 1) & 1) + 4 * (wave & 1)) * vst;
         v_st = vst;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) v_lane[j] = (lane + 64 * j < p.d ? lane + 64 * j : 0) * 4;
+        for (int j = 0; j < NJ; ++j) {
+            const int dim = dim_of(wave, lane, j);
+            v_lane[j] = (dim < p.d ? dim : 0) * 4;
+        }
     }
 
     // Rows key0 .. key0 + 31 of a KV head, ending with the last key (rows past
@@ -216,21 +188,21 @@ struct SplitTile {
 #pragma unroll
                 for (int i = 0; i < NK; ++i)
                     kr[i] = __builtin_bit_cast(
-                        float4, __builtin_amdgcn_raw_buffer_load_b128(range, k_lane, i * k_step, 0));
+                        float4, __builtin_amdgcn_raw_buffer_load_b128(range, k_lane[i % NC], i / NC * k_step, 0));
             } else {
                 // The range check is on the lane's offset, so all of it goes there.
 #pragma unroll
                 for (int i = 0; i < NK; ++i)
                     kr[i] = __builtin_bit_cast(
-                        float4, __builtin_amdgcn_raw_buffer_load_b128(range, k_lane + i * k_step, 0, 0));
+                        float4, __builtin_amdgcn_raw_buffer_load_b128(range, k_lane[i % NC] + i / NC * k_step, 0, 0));
             }
         } else if (ok) {
-            const int rs = lane / LPR, c = (lane % LPR) * 4;
 #pragma unroll
             for (int i = 0; i < NK; ++i) {
-                int key = key0 + 8 * wave + rs + RPI * i;
+                int key = key0 + KR * wave + row_of(lane) + RPI * (i / NC);
                 if (key > p.Tk - 1) key = p.Tk - 1;
                 const float* a = kb + key * p.k.st;
+                const int c = col_of(lane, i % NC);
                 float t[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) t[j] = a[(c + j < p.d ? c + j : 0) * p.k.sd];
@@ -240,23 +212,22 @@ struct SplitTile {
     }
 
     __device__ __forceinline__ void store_k(char* ks, int wave, int lane) const {
-        const int rs = lane / LPR, i4 = lane % LPR;
-        const int c8 = i4 >> 1;            // 8-dim chunk 2t + h
-        char* base = ks + c8 * 512 + (i4 & 1) * 8;
 #pragma unroll
         for (int i = 0; i < NK; ++i) {
-            const int r = 8 * wave + rs + RPI * i;
+            const int c4 = col_of(lane, i % NC) >> 2, c8 = c4 >> 1;   // 8-dim chunk 2t + h
+            const int r = KR * wave + row_of(lane) + RPI * (i / NC);
             uint2 h, m, l;
             split3(kr[i].x, kr[i].y, h.x, m.x, l.x);
             split3(kr[i].z, kr[i].w, h.y, m.y, l.y);
-            char* a = base + ((r ^ (c8 & 15)) << 4);
+            char* a = ks + c8 * 512 + (c4 & 1) * 8 + ((r ^ (c8 & 15)) << 4);
             *reinterpret_cast<uint2*>(a) = h;
             *reinterpret_cast<uint2*>(a + K_PLANE) = m;
             *reinterpret_cast<uint2*>(a + 2 * K_PLANE) = l;
         }
     }
 
-    // Wave w reads the 8 keys of (step s, lane half h) = (w / 2, w % 2).
+    // Wave w reads the 8 keys of (step s, lane half h) = (w / 2 % 2, w % 2); with
+    // 8 waves, waves 4-7 the second half of the dims.
     __device__ __forceinline__ void load_v(const PrefillParams& p, const float* vb, int key0,
                                            int wave, int lane, bool ok) {
         if (VEC) {
@@ -277,7 +248,7 @@ struct SplitTile {
                             range, v_lane[j] + v_row0 + (8 * (i >> 2) + (i & 3)) * v_st, 0, 0));
             }
         } else if (ok) {
-            const int k0 = key0 + 16 * (wave >> 1) + 4 * (wave & 1);
+            const int k0 = key0 + 16 * ((wave >> 1) & 1) + 4 * (wave & 1);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 int key = k0 + 8 * (i >> 2) + (i & 3);
@@ -285,7 +256,7 @@ struct SplitTile {
                 const float* a = vb + key * p.v.st;
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
-                    const int dim = lane + 64 * j;
+                    const int dim = dim_of(wave, lane, j);
                     vr[j][i] = a[(dim < p.d ? dim : 0) * p.v.sd];
                 }
             }
@@ -295,14 +266,14 @@ struct SplitTile {
     __device__ __forceinline__ void store_v(char* vs, int wave, int lane) const {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const int dim = lane + 64 * j;
-            if (64 * (j + 1) > D && dim >= D) continue;
+            const int dim = dim_of(wave, lane, j);
+            if (64 * (j + 1) > VD && lane + 64 * j >= VD) continue;
             uint4 h, m, l;
             split3(vr[j][0], vr[j][1], h.x, m.x, l.x);
             split3(vr[j][2], vr[j][3], h.y, m.y, l.y);
             split3(vr[j][4], vr[j][5], h.z, m.z, l.z);
             split3(vr[j][6], vr[j][7], h.w, m.w, l.w);
-            char* a = vs + (((dim >> 5) * 2 + (wave >> 1)) * 64 + (wave & 1) * 32 + (dim & 31)) * 16;
+            char* a = vs + (((dim >> 5) * 2 + ((wave >> 1) & 1)) * 64 + (wave & 1) * 32 + (dim & 31)) * 16;
             *reinterpret_cast<uint4*>(a) = h;
             *reinterpret_cast<uint4*>(a + V_PLANE) = m;
             *reinterpret_cast<uint4*>(a + 2 * V_PLANE) = l;
@@ -310,18 +281,18 @@ struct SplitTile {
     }
 };
 
-// One 32-row unit over key tiles [t0, t1) in plain f32 MFMAs on operands read
-// from global memory: the arithmetic for inputs outside the range in which the
+// One 32-row unit (its output dims dim0 .. dim0 + 32 NB - 1) over key tiles
+// [t0, t1) in plain f32 MFMAs on operands read from global memory: the arithmetic for inputs outside the range in which the
 // three bf16 parts hold all 24 bits.  Slow, and rare.  Everything it needs is
 // derived here from a few opaque scalars, so that nothing of it is computed
 // ahead of, or kept in registers across, the main loop.
-template <int D, bool CAUSAL>
+template <int D, int NB, bool CAUSAL>
 __device__ __forceinline__ void unit_f32(const PrefillParams& p, int head, int unit, int t0, int t1,
-                                         floatx16 (&o)[D / 32], float& m_run, float& l_run) {
-    constexpr int NB = D / 32;
+                                         int dim0, floatx16 (&o)[NB], float& m_run, float& l_run) {
     int tid = threadIdx.x;
     float zero = 0.f;
-    asm volatile("" : "+v"(tid), "+v"(zero), "+s"(head), "+s"(unit), "+s"(t0), "+s"(t1));
+    asm volatile("" : "+v"(tid), "+v"(zero), "+s"(head), "+s"(unit), "+s"(t0), "+s"(t1),
+                 "+s"(dim0));
     const int l32 = tid & 31, half = (tid >> 5) & 1;
     const int bi = head / p.Hkv, kvh = head % p.Hkv;
     const int qrow = unit / p.G * 32 + l32;
@@ -376,7 +347,7 @@ __device__ __forceinline__ void unit_f32(const PrefillParams& p, int head, int u
             const float* vp = vb + (int64_t)(key < p.Tk ? key : 0) * p.v.st;
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                const int dim = 32 * b + l32;
+                const int dim = dim0 + 32 * b + l32;
                 const float vx = key < p.Tk && dim < p.d ? vp[dim * p.v.sd] : 0.f;
                 o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx, pr, o[b], 0, 0, 0);
             }
@@ -690,7 +661,7 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
 #pragma unroll
         for (int r = 0; r < 16; ++r) o_code = max(o_code, range_code(o[b][r]));
     if (__builtin_amdgcn_ballot_w64(q_code > kQueryCodes || o_code >= kResultCodes) != 0)
-        unit_f32<D, CAUSAL>(p, head, unit, t0, min(t1, wave_tiles), o, m_run, l_run);
+        unit_f32<D, NB, CAUSAL>(p, head, unit, t0, min(t1, wave_tiles), 0, o, m_run, l_run);
 
     float l_tot = pair_sum(l_run);
     if constexpr (SPLIT) {
@@ -789,27 +760,33 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
     }
 }
 
-// Head dims 129..256, padded to 256.  Q^T and O^T of 256 dims do not fit one
-// wave's registers beside its K/V operands, so every 32-row unit is served
-// by two waves, one per half of the head dim: wave (unit u, half h) holds
-// Q^T and O^T of dims [128h, 128h + 128).  Per 32-key tile each wave computes
-// the partial S^T over its dims (the d = 128 kernel's 64 MFMAs), the two swap
-// their partials through the K/V stage that is idle during the tile, and
-// both add them -- a + b == b + a, so the pair holds the same S bit for bit
-// and runs the same online softmax -- then each accumulates its half of
-// O^T = V^T P^T.  8 waves (4 units, the 4 (row block, query head) units of
-// the d = 128 kernel) per workgroup and one workgroup per CU: two stages of
-// 32 keys x 256 dims of K and V take 134 KB of LDS.  K/V come from HBM once
-// per KV head and workgroup step, as at d <= 128.
-template <bool CAUSAL>
+// Head dims above 128: NW waves of a workgroup of 8 serve one 32-row unit, each
+// with DW of its dims -- Q^T and O^T of DW <= 128 dims are what one wave's
+// registers hold -- so a workgroup takes 8 / NW units (the (row block, query
+// head) units of one KV head, as at d <= 128), which share every staged and
+// split K/V tile.  Per 32-key tile each wave computes the partial S^T over its
+// dims, leaves it in LDS, and every wave of the unit adds the NW partials in
+// wave order: they hold the same S bit for bit and run the same online softmax;
+// then each accumulates its DW dims of O^T = V^T P^T.
+//
+// One workgroup per CU.  Up to 256 dims K and V have a buffer each, replaced a
+// phase apart as in the d <= 128 kernel (two barriers per tile); at 512 a tile
+// of either is 98 KB, so both go through one buffer (four barriers).  The low
+// parts of Q's last steps stay in LDS.
+template <int DW, int NW, bool CAUSAL, bool VEC>
 __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParams p) {
-    constexpr int D = 256, DH = D / 2;
-    constexpr int KS = D + 4, VS = D + 8;
-    constexpr int STAGE = 32 * KS + 32 * VS;
-    constexpr int NB = DH / 32;          // 32-wide output column blocks per wave
-    constexpr int XW = 16 * 64;          // floats of one wave's partial S^T
-    static_assert(8 * XW <= STAGE, "the partials fit the idle stage");
-    __shared__ __attribute__((aligned(16))) float lds[2 * STAGE];
+    constexpr int D = DW * NW, U = 8 / NW;
+    using Tile = SplitTile<D, VEC, 8>;
+    constexpr int KP = Tile::K_PLANE;
+    constexpr int NB = DW / 32;          // 32-wide output column blocks per wave
+    constexpr int NT = DW / 16;          // 16-dim steps of a wave's partial S^T
+    constexpr int NQL = 4;               // steps whose low parts of Q are in LDS
+    constexpr bool ONE = NW > 2;         // K and V share a buffer
+    __shared__ __attribute__((aligned(16))) char lds[(ONE ? 3 : 6) * KP + 8 * 4096 + 8 * NQL * 1024];
+    char* const Ks = lds;
+    char* const Vs = ONE ? lds : lds + 3 * KP;
+    char* const Xs = Vs + 3 * KP;        // partial S^T, 4 KB per wave
+    char* const Qs = Xs + 8 * 4096;
 
     const int x = blockIdx.x & 7, q = blockIdx.x >> 3, S = gridDim.x >> 3;
 
@@ -821,12 +798,12 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
     if (st == 2) continue;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const int dh = wave >> 2;            // head-dim half of this wave
+    const int dq = wave / U;             // which DW dims this wave holds
     const int bi = head / p.Hkv, kvh = head % p.Hkv;
 
-    const int unit = wgi * 4 + (wave & 3);
+    const int unit = wgi * U + wave % U;
     const bool active = unit < p.n_units;
     const int rb = active ? unit / p.G : 0;
     const int g = active ? unit % p.G : 0;
@@ -835,7 +812,7 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
     const int qrow = row0 + l32;
 
     const int n_kt = (p.Tk + 31) >> 5;
-    int last_unit = wgi * 4 + 3;
+    int last_unit = wgi * U + U - 1;
     if (last_unit > p.n_units - 1) last_unit = p.n_units - 1;
     const int wg_last_key = last_visible_key(p, last_unit / p.G, CAUSAL);
     int n_tiles = wg_last_key < 0 ? 0 : (wg_last_key >> 5) + 1;
@@ -843,22 +820,40 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
     const int wave_last_key = last_visible_key(p, rb, CAUSAL);
     const int wave_tiles = active ? (wave_last_key < 0 ? 0 : (wave_last_key >> 5) + 1) : 0;
 
-    // Q^T fragment: qf[s] = Q[qrow][dh*128 + half*64 + s] * scale*log2(e)
-    float qf[DH / 2];
-    {
-        const float* qp = p.q.p + bi * p.q.sb + hq * p.q.sh + (int64_t)qrow * p.q.st;
-        const bool rok = active && qrow < p.Tq;
+    // Q^T: three bf16 parts of Q[qrow][dq*DW + 16t + 8*half + 0..7] * scale*log2(e)
+    short8 qf[2][NT], ql[NT - NQL];
+    char* const qls = Qs + (wave * NQL * 64 + lane) * 16;
+    const float* qp = p.q.p + bi * p.q.sb + hq * p.q.sh + (int64_t)qrow * p.q.st;
+    const bool rok = active && qrow < p.Tq;
+    uint32_t q_code = 0;
 #pragma unroll
-        for (int s4 = 0; s4 < DH / 8; ++s4) {
-            const int c = dh * DH + half * (DH / 2) + 4 * s4;
-            const float4 t = (rok && c < p.d) ? *reinterpret_cast<const float4*>(qp + c)
-                                              : make_float4(0.f, 0.f, 0.f, 0.f);
-            qf[4 * s4 + 0] = t.x * p.qscale;
-            qf[4 * s4 + 1] = t.y * p.qscale;
-            qf[4 * s4 + 2] = t.z * p.qscale;
-            qf[4 * s4 + 3] = t.w * p.qscale;
+    for (int t = 0; t < NT; ++t) {
+        const int c = dq * DW + 16 * t + 8 * half;
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+            const float4 t4 = (rok && c + j < p.d) ? *reinterpret_cast<const float4*>(qp + c + j)
+                                                   : make_float4(0.f, 0.f, 0.f, 0.f);
+            x[j] = t4.x; x[j + 1] = t4.y; x[j + 2] = t4.z; x[j + 3] = t4.w;
         }
+        uint4 h, m, l;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            x[j] *= p.qscale;
+            q_code = max(q_code, range_code(x[j]));
+        }
+        split3(x[0], x[1], h.x, m.x, l.x);
+        split3(x[2], x[3], h.y, m.y, l.y);
+        split3(x[4], x[5], h.z, m.z, l.z);
+        split3(x[6], x[7], h.w, m.w, l.w);
+        qf[0][t] = __builtin_bit_cast(short8, h);
+        qf[1][t] = __builtin_bit_cast(short8, m);
+        if (t < NT - NQL) ql[t < NT - NQL ? t : 0] = __builtin_bit_cast(short8, l);
+        else *reinterpret_cast<uint4*>(qls + (t - (NT - NQL)) * 1024) = l;
     }
+    // A query whose parts lose bits makes every S of its row NaN, so that all
+    // waves of the unit see it in their results.
+    if (q_code > kQueryCodes) qf[0][0] = short8{0x7fc0, 0x7fc0, 0x7fc0, 0x7fc0, 0x7fc0, 0x7fc0, 0x7fc0, 0x7fc0};
 
     const float* kb = p.k.p + bi * p.k.sb + kvh * p.k.sh;
     const float* vb = p.v.p + bi * p.v.sb + kvh * p.v.sh;
@@ -872,14 +867,17 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
 
     // Second items of causal pairs walk their key tiles backwards, as in the
     // d <= 128 kernel (a head's K/V tiles stay in the XCD's L2: 688 -> 260 MB
-    // read at B = 1, H = 16, T = 4096).
+    // read at B = 1, H = 16, T = 4096, d = 256).
     const bool rev = p.pairing && (j & 1);
     const int kstep = rev ? -1 : 1;
     const int kfirst = rev ? n_tiles - 1 : 0;
-    TileLoader<D, true, 512> ld;
+    Tile ld;
+    ld.init(p, wave, lane);
     if (n_tiles > 0) {
-        ld.load(p, kb, vb, kfirst * 32, tid);
-        ld.store(lds, lds + 32 * KS, tid);
+        ld.load_k(p, kb, kfirst * 32, wave, lane, true);
+        ld.load_v(p, vb, kfirst * 32, wave, lane, true);
+        ld.store_k(Ks, wave, lane);
+        if (!ONE) ld.store_v(Vs, wave, lane);
     }
     __syncthreads();
 
@@ -887,53 +885,80 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
         const int kt = kfirst + kstep * it;
         const bool has_next = it + 1 < n_tiles;
         const bool mine = kt < wave_tiles;
-        const float* Ks = lds + (it & 1) * STAGE;
-        const float* Vs = Ks + 32 * KS;
-        float* other = lds + ((it + 1) & 1) * STAGE;   // idle until the next tile's store
+        if (!ONE) ld.load_k(p, kb, (kt + kstep) * 32, wave, lane, has_next);
         floatx16 s;
+        const float m_use = (m_run == kNegInf) ? 0.f : m_run;
         if (mine) {
-            // Partial S^T = K Q^T over this wave's 128 dims, log2 domain.
+            // Partial S^T = K Q^T over this wave's dims, log2 domain.
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] = 0.f;
-            const float* krow = Ks + l32 * KS + dh * DH + half * (DH / 2);
+            const char* kw = Ks + dq * NT * 1024;
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int t = 0; t < DH / 8; ++t) {
-                const float4 kq = *reinterpret_cast<const float4*>(krow + 4 * t);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.x, qf[4 * t + 0], s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.y, qf[4 * t + 1], s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.z, qf[4 * t + 2], s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kq.w, qf[4 * t + 3], s, 0, 0, 0);
+            for (int t = 0; t < NT; ++t) {
+                const char* a = kw + t * 1024 + half * 512 + ((l32 ^ ((2 * (dq * NT + t) + half) & 15)) << 4);
+                const short8 kh = *reinterpret_cast<const short8*>(a);
+                const short8 km = *reinterpret_cast<const short8*>(a + KP);
+                const short8 kl = *reinterpret_cast<const short8*>(a + 2 * KP);
+                s = mfma_bf16(kl, qf[0][t], s);
+                s = mfma_bf16(kh, t < NT - NQL ? ql[t < NT - NQL ? t : 0]
+                                               : *reinterpret_cast<const short8*>(
+                                                     qls + (t - (NT - NQL)) * 1024), s);
+                s = mfma_bf16(km, qf[1][t], s);
+                s = mfma_bf16(km, qf[0][t], s);
+                s = mfma_bf16(kh, qf[1][t], s);
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            for (int t = 0; t < NT; ++t) {
+                const char* a = kw + t * 1024 + half * 512 + ((l32 ^ ((2 * (dq * NT + t) + half) & 15)) << 4);
+                s = mfma_bf16(*reinterpret_cast<const short8*>(a), qf[0][t], s);
+            }
+            // Schedule: the operands of a step are read one step ahead.
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
 #pragma unroll
-            for (int i = 0; i < DH / 8 - 4; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            for (int t = 0; t < NT - 1; ++t) {
+                if (t + 1 < NT - NQL) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                else __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 5, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 5, 0);
+#pragma unroll
+            for (int t = 0; t < NT - 2; ++t) {
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
             __builtin_amdgcn_s_setprio(0);
             // This wave's partial, register-group major (each store one
             // contiguous, conflict-free 1 KB wave access).
-            float* xo = other + wave * XW + 4 * lane;
+            char* xo = Xs + wave * 4096 + lane * 16;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                *reinterpret_cast<float4*>(xo + 256 * i) =
+                *reinterpret_cast<float4*>(xo + 1024 * i) =
                     make_float4(s[4 * i], s[4 * i + 1], s[4 * i + 2], s[4 * i + 3]);
         }
-        if (has_next) ld.load(p, kb, vb, (kt + kstep) * 32, tid);
-        __syncthreads();   // partials visible
+        __syncthreads();   // partials visible, K read (and V visible)
+        if (ONE) {
+            ld.store_v(Vs, wave, lane);
+            ld.load_k(p, kb, (kt + kstep) * 32, wave, lane, has_next);
+        } else {
+            if (has_next) ld.store_k(Ks, wave, lane);
+            ld.load_v(p, vb, (kt + kstep) * 32, wave, lane, has_next);
+        }
         if (mine) {
-            // Add the partner's partial: wave w pairs with wave w ^ 4.
-            const float* xi = other + (wave ^ 4) * XW + 4 * lane;
+            // S^T - m: the unit's partials in wave order.
+            const char* xi = Xs + (wave % U) * 4096 + lane * 16;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float4 t = *reinterpret_cast<const float4*>(xi + 256 * i);
-                s[4 * i] += t.x;
-                s[4 * i + 1] += t.y;
-                s[4 * i + 2] += t.z;
-                s[4 * i + 3] += t.w;
+                float4 a = *reinterpret_cast<const float4*>(xi + 1024 * i);
+#pragma unroll
+                for (int w = 1; w < NW; ++w) {
+                    const float4 t = *reinterpret_cast<const float4*>(xi + w * U * 4096 + 1024 * i);
+                    a.x += t.x; a.y += t.y; a.z += t.z; a.w += t.w;
+                }
+                s[4 * i] = a.x - m_use; s[4 * i + 1] = a.y - m_use;
+                s[4 * i + 2] = a.z - m_use; s[4 * i + 3] = a.w - m_use;
             }
             const int key0 = kt * 32;
             const bool need_mask = (key0 + 32 > p.Tk) || (CAUSAL && key0 + 31 > row0 + p.q_offset);
@@ -945,57 +970,86 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
                     s[r] = vis ? s[r] : kNegInf;
                 }
             }
-            // Online softmax with the lazy rescale of the d <= 128 kernel; both
-            // waves of the pair take the same decisions on the same values.
+            // Online softmax with the lazy rescale of the d <= 128 kernel; all
+            // waves of the unit take the same decisions on the same values.
             float mt = s[0];
 #pragma unroll
             for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
             mt = pair_max(mt);
-            if (__builtin_amdgcn_ballot_w64(mt > m_run + 8.f) != 0) {
-                const float m_new = fmaxf(m_run, mt);
-                const float alpha = fast_exp2(m_run - ((m_new == kNegInf) ? 0.f : m_new));
+            if (__builtin_amdgcn_ballot_w64(mt > (m_run == kNegInf ? kNegInf : 8.f)) != 0) {
+                const float m_new = fmaxf(m_run, mt + m_use);
+                const float n_use = (m_new == kNegInf) ? 0.f : m_new;
+                const float alpha = fast_exp2(m_run - n_use);
                 l_run *= alpha;
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] -= n_use - m_use;
                 m_run = m_new;
             }
-            const float m_use = (m_run == kNegInf) ? 0.f : m_run;
             float ls = 0.f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                s[r] = fast_exp2(s[r] - m_use);
+                s[r] = fast_exp2(s[r]);
                 ls += s[r];
             }
             l_run += ls;
-
-            // O^T += V^T P^T over this wave's 128 output dims.
+        }
+        if (ONE) __syncthreads();   // V visible
+        if (mine) {
+            // O^T += V^T P^T over this wave's output dims.
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float* vrow = Vs + (8 * (r >> 2) + 4 * half + (r & 3)) * VS + dh * DH + l32;
+            for (int st = 0; st < 2; ++st) {
+                uint4 h, m, l;
+                split3(s[8 * st + 0], s[8 * st + 1], h.x, m.x, l.x);
+                split3(s[8 * st + 2], s[8 * st + 3], h.y, m.y, l.y);
+                split3(s[8 * st + 4], s[8 * st + 5], h.z, m.z, l.z);
+                split3(s[8 * st + 6], s[8 * st + 7], h.w, m.w, l.w);
+                const short8 ph = __builtin_bit_cast(short8, h), pm = __builtin_bit_cast(short8, m),
+                             pl = __builtin_bit_cast(short8, l);
 #pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * b], s[r], o[b], 0, 0, 0);
+                for (int b = 0; b < NB; ++b) {
+                    const char* a = Vs + (((dq * NB + b) * 2 + st) * 64 + lane) * 16;
+                    const short8 vh = *reinterpret_cast<const short8*>(a);
+                    const short8 vm = *reinterpret_cast<const short8*>(a + KP);
+                    const short8 vl = *reinterpret_cast<const short8*>(a + 2 * KP);
+                    o[b] = mfma_bf16(vl, ph, o[b]);
+                    o[b] = mfma_bf16(vh, pl, o[b]);
+                    o[b] = mfma_bf16(vm, pm, o[b]);
+                    o[b] = mfma_bf16(vm, ph, o[b]);
+                    o[b] = mfma_bf16(vh, pm, o[b]);
+                    o[b] = mfma_bf16(vh, ph, o[b]);
+                }
             }
-            constexpr int NVR = 16 * NB / 2;
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-#pragma unroll
-            for (int i = 0; i < NVR - 4; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            for (int i = 0; i < 2 * NB - 1; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
             __builtin_amdgcn_s_setprio(0);
         }
-        if (has_next) {
-            __syncthreads();   // every partial read before the stage is refilled
-            ld.store(other, other + 32 * KS, tid);
+        __syncthreads();   // V and the partials are read (and the next K visible)
+        if (ONE) {
+            if (has_next) ld.store_k(Ks, wave, lane);
+            ld.load_v(p, vb, (kt + kstep) * 32, wave, lane, has_next);
+            __syncthreads();   // the next K is visible
+        } else {
+            if (has_next) ld.store_v(Vs, wave, lane);
         }
-        __syncthreads();
     }
+
+    uint32_t o_code = 0;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_code = max(o_code, range_code(o[b][r]));
+    if (__builtin_amdgcn_ballot_w64(o_code >= kResultCodes) != 0)
+        unit_f32<D, NB, CAUSAL>(p, head, unit, 0, wave_tiles, dq * DW, o, m_run, l_run);
 
     const float l_tot = pair_sum(l_run);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -1005,7 +1059,7 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
         for (int b = 0; b < NB; ++b) {
 #pragma unroll
             for (int qq = 0; qq < 4; ++qq) {
-                const int c = dh * DH + 32 * b + 8 * qq + 4 * half;
+                const int c = dq * DW + 32 * b + 8 * qq + 4 * half;
                 if (c < p.d)
                     *reinterpret_cast<float4*>(op + c) =
                         make_float4(o[b][4 * qq] * inv, o[b][4 * qq + 1] * inv,
@@ -1037,6 +1091,19 @@ void residency(int& cus, int& per_cu) {
     }
     cus = c;
     per_cu = k;
+}
+
+int device_cus() {
+    static std::atomic<int> cached[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+    int c = cached[dev].load(std::memory_order_relaxed);
+    if (c == 0) {
+        if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c < 8)
+            c = 256;
+        cached[dev].store(c, std::memory_order_relaxed);
+    }
+    return c;
 }
 
 // One resident wave of persistent workgroups: k per CU on every CU (an
@@ -1094,27 +1161,17 @@ hipError_t launch_t(PrefillParams p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Head dims 129..256: the wave-pair kernel, one workgroup of 8 waves per CU.
-template <bool CAUSAL>
-hipError_t launch_wide_t(PrefillParams p, hipStream_t stream) {
-    constexpr auto kernel = prefill_wide_kernel<CAUSAL>;
-    static std::atomic<int> cached_cus[64], cached_per[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    int cus = cached_cus[dev].load(std::memory_order_acquire);
-    int k_max = cached_per[dev].load(std::memory_order_relaxed);
-    if (cus == 0 || k_max == 0) {
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus < 8)
-            cus = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k_max, kernel, 512, 0) != hipSuccess ||
-            k_max < 1)
-            k_max = 1;
-        cached_per[dev].store(k_max, std::memory_order_relaxed);
-        cached_cus[dev].store(cus, std::memory_order_release);
-    }
-    const int S = persistent_slots(p, CAUSAL, cus, k_max);
-    hipLaunchKernelGGL(kernel, dim3(8 * S), dim3(512), 0, stream, p);
+// Head dims 129..512: one workgroup of 8 waves per CU.
+template <int DW, int NW, bool VEC = true>
+hipError_t launch_wide_d(PrefillParams p, bool causal, hipStream_t stream) {
+    constexpr int U = 8 / NW;
+    p.n_wg = (p.n_units + U - 1) / U;
+    p.total = p.B * p.Hkv * p.n_wg;
+    const int S = persistent_slots(p, causal, device_cus(), 1);
+    if (causal)
+        hipLaunchKernelGGL((prefill_wide_kernel<DW, NW, true, VEC>), dim3(8 * S), dim3(512), 0, stream, p);
+    else
+        hipLaunchKernelGGL((prefill_wide_kernel<DW, NW, false, VEC>), dim3(8 * S), dim3(512), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -1141,19 +1198,6 @@ void derive_schedule(PrefillParams& p) {
     p.n_units = p.G * p.n_rb;
     p.n_wg = (p.n_units + 3) / 4;
     p.total = p.B * p.Hkv * p.n_wg;
-}
-
-int device_cus() {
-    static std::atomic<int> cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    int c = cached[dev].load(std::memory_order_relaxed);
-    if (c == 0) {
-        if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c < 8)
-            c = 256;
-        cached[dev].store(c, std::memory_order_relaxed);
-    }
-    return c;
 }
 
 }  // namespace
@@ -1224,19 +1268,27 @@ PrefillSplit prefill_split_plan(PrefillParams& p, bool causal, bool vec) {
     return r;
 }
 
+// The vector loads of a K/V tile hold its row offsets in 32 bits.
+static bool row_offsets_fit(const PrefillParams& p) {
+    return p.k.st >= 0 && p.k.st < kMaxTileStride && p.v.st >= 0 && p.v.st < kMaxTileStride;
+}
+
 hipError_t launch_prefill_wide(PrefillParams p, bool causal, hipStream_t stream) {
     derive_schedule(p);
     if (p.total == 0) return hipSuccess;
-    if (p.d <= 128 || p.d > 256) return hipErrorInvalidValue;
-    return causal ? launch_wide_t<true>(p, stream) : launch_wide_t<false>(p, stream);
+    if (p.d <= 128 || p.d > 512) return hipErrorInvalidValue;
+    if (!row_offsets_fit(p))
+        return p.d <= 256 ? launch_wide_d<128, 2, false>(p, causal, stream) : hipErrorInvalidValue;
+    if (p.d <= 192) return launch_wide_d<96, 2>(p, causal, stream);
+    if (p.d <= 256) return launch_wide_d<128, 2>(p, causal, stream);
+    if (p.d <= 384) return launch_wide_d<96, 4>(p, causal, stream);
+    return launch_wide_d<128, 4>(p, causal, stream);
 }
 
 hipError_t launch_prefill(PrefillParams p, bool causal, bool vec, hipStream_t stream) {
     derive_schedule(p);
     if (p.total == 0) return hipSuccess;
-    // The vector loads of a K/V tile hold its row offsets in 32 bits.
-    constexpr int64_t kMaxRowStride = 1 << 24;
-    vec = vec && p.k.st >= 0 && p.k.st < kMaxRowStride && p.v.st >= 0 && p.v.st < kMaxRowStride;
+    vec = vec && row_offsets_fit(p);
     switch (prefill_padded_dim(p.d)) {
         case 32: return launch_d<32>(p, causal, vec, stream);
         case 64: return launch_d<64>(p, causal, vec, stream);

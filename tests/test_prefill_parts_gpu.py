@@ -54,6 +54,43 @@ def test_tile_edges(heads, d, tq, tk, causal):
     check64(run(q, k, v, causal, tk - tq), attend64(q, k, v, causal, tk - tq))
 
 
+# More 32-row units than two per CU: the 8-wave kernel (at 512 dims with K and V
+# in one buffer); rows that are not whole units, tails of one key, padded dims.
+@pytest.mark.parametrize("d", [132, 192, 196, 256, 260, 384, 388, 512])
+@pytest.mark.parametrize("hq,hkv,tq,tk,causal", [(140, 140, 97, 129, True), (140, 20, 97, 31, False),
+                                                 (75, 75, 225, 225, True)])
+def test_tile_edges_above_128_dims(d, hq, hkv, tq, tk, causal):
+    q, k, v = draw(d + tq, 1, hq, hkv, tq, tk, d)
+    check64(run(q, k, v, causal, tk - tq), attend64(q, k, v, causal, tk - tq))
+
+
+@pytest.mark.parametrize("d", [256, 512])
+@pytest.mark.parametrize("qs,ks,vs", [(1.0, 1.0, 1e-37), (1e-30, 1e30, 1.0), (1e30, 1e-30, 1.0)])
+def test_magnitudes_above_128_dims(d, qs, ks, vs):
+    q, k, v = draw(17, 1, 140, 140, 97, 129, d)
+    q[..., d // 2:] *= np.float32(qs)      # half of the dims: one wave sees them, all must know
+    k[..., d // 2:] *= np.float32(ks)
+    v *= np.float32(vs)
+    ref = attend64(q, k, v, True, 32)
+    scale = 1 / np.abs(ref).max()
+    check64(run(q, k, v, True, 32).astype(np.float64) * scale, ref * scale)
+
+
+@pytest.mark.parametrize("d", [256, 512])
+def test_infinities_above_128_dims(d):
+    q, k, v = draw(18, 1, 140, 140, 97, 129, d)
+    q[:, 3] = np.abs(q[:, 3]) + np.float32(0.01)
+    k[:, 3, 50] = -np.inf
+    v[0, 5, 70, d - 1] = np.inf
+    o = run(q, k, v, False)
+    k[:, 3, 50] = -1e30
+    ref = attend64(q, k, v, False)
+    assert np.isposinf(o[0, 5, :, d - 1]).all()
+    check64(o[0, 5, :, :d - 1], ref[0, 5, :, :d - 1])
+    others = [h for h in range(140) if h != 5]
+    check64(o[:, others], ref[:, others])
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("qs,ks,vs", [(1.0, 1.0, 1e-37), (1.0, 1.0, 1e34), (1e-30, 1e30, 1.0),
                                       (1e30, 1e-30, 1.0), (1e-36, 1e36, 1e-36)])
