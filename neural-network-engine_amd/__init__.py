@@ -25,13 +25,18 @@ There is no CPU path: if the HIP library is missing, importing works but every
 call raises.
 """
 import ctypes
+import functools
+import importlib.machinery
+import importlib.util
 import math
 import os
+import types
 
 import numpy as np
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "lib", "libnne_attn.so")
+CALL_PATH = os.path.join(_PKG, "lib", "nne_pycall.so")
 
 NNE_OK, NNE_EINVAL, NNE_ESHAPE, NNE_ECAPACITY, NNE_EHIP = 0, 1, 2, 3, 4
 
@@ -60,10 +65,13 @@ _ERRORS = {NNE_EINVAL: InvalidArgument, NNE_ESHAPE: ShapeMismatch,
            NNE_ECAPACITY: CapacityError, NNE_EHIP: GpuError}
 
 _lib = None
+_calls = None       # the step calls on the native path (csrc/pycall.cpp)
 
-_i64p = ctypes.POINTER(ctypes.c_int64)
-_i32p = ctypes.POINTER(ctypes.c_int32)
+# Arrays cross as plain addresses: converting to a typed ctypes pointer costs
+# more than the rest of an argument's conversion.  (c_void_p takes ctypes
+# arrays, pointers and byref objects too.)
 _vp = ctypes.c_void_p
+_i64p = _i32p = _vp
 
 
 class NneWorkspace(ctypes.Structure):
@@ -78,6 +86,7 @@ class NneWorkspaceSize(ctypes.Structure):
 
 
 _wsp = ctypes.POINTER(NneWorkspace)
+_i64x4 = ctypes.c_int64 * 4
 _wszp = ctypes.POINTER(NneWorkspaceSize)
 
 # exported symbol -> (restype, argtypes); mirrors include/nne_attn.h
@@ -149,7 +158,7 @@ SIGNATURES = {
 
 def lib():
     """The loaded HIP library; raises if it has not been built."""
-    global _lib
+    global _lib, _calls
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise GpuError("HIP attention library not built: %s is missing "
@@ -159,8 +168,36 @@ def lib():
             fn = getattr(l, name)
             fn.restype = res
             fn.argtypes = args
+        _calls = _native_calls(l)
         _lib = l
     return _lib
+
+
+def _native_calls(l):
+    """The ABI functions of a decode or prefill step, called through the
+    nne_pycall module: it takes tuples, addresses and numpy arrays as they are,
+    where ctypes spent 4-5 us converting the arguments of a call."""
+    if not os.path.exists(CALL_PATH):
+        raise GpuError("native call module not built: %s is missing "
+                       "(run neural-network-engine_amd/build.py)" % CALL_PATH)
+    loader = importlib.machinery.ExtensionFileLoader("nne_pycall", CALL_PATH)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("nne_pycall", loader))
+
+    def call(fn, name):
+        return functools.partial(fn, ctypes.cast(getattr(l, name), ctypes.c_void_p).value)
+
+    return types.SimpleNamespace(
+        flash=call(mod.flash, "nne_flash_attention_forward_ws"),
+        attention=call(mod.attention, "nne_attention_forward_ws"),
+        decode_attention=call(mod.decode_attention, "nne_decode_attention"),
+        decode_step=call(mod.decode_step, "nne_decode_step"),
+        qkv_rope=call(mod.qkv_rope, "nne_qkv_rope_ws"))
+
+
+def _native():
+    if _lib is None:
+        lib()
+    return _calls
 
 
 def check(rc):
@@ -170,14 +207,19 @@ def check(rc):
 
 
 def _i64(vals):
-    arr = (ctypes.c_int64 * 4)(*[int(x) for x in vals])
-    return arr
+    try:
+        return _i64x4(*vals)
+    except TypeError:      # not Python ints
+        return _i64x4(*[int(x) for x in vals])
 
 
 def _stream(stream=None):
+    """The stream's handle as an int (the current device's current stream by
+    default; its raw handle, since wrapping it in a Stream object costs 3 us)."""
+    if stream is not None:
+        return stream.cuda_stream
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def release_stream(stream=None):
@@ -228,13 +270,16 @@ class Workspace:
             w.counters, w.n_counters = self.counters.data_ptr(), self.counters.numel()
         return ctypes.byref(w), w
 
+    def _args(self):
+        """The fields of nne_workspace_t, as the native calls take them."""
+        r, c = self.records, self.counters
+        return (0 if r is None else r.data_ptr(), 0 if r is None else r.numel(),
+                0 if c is None else c.data_ptr(), 0 if c is None else c.numel())
+
 
 def _ws_arg(workspace, size, stream):
-    """(pointer argument, keep-alive) for an optional Workspace."""
-    if workspace is None:
-        return None, None
-    workspace.reserve(size, stream)
-    return workspace.struct()
+    """The native calls' argument for a Workspace grown to ``size``."""
+    return workspace.reserve(size, stream)._args()
 
 
 def _require_f32_cuda(*ts):
@@ -266,20 +311,18 @@ def flash_attention_forward(q, k, v, is_causal, scale=None, block_size_r=64, blo
     q, k, v: float32 CUDA tensors [B, H, T, d] with any strides.  Returns a new
     contiguous [B, H, Tq, d] tensor (or fills ``out``).  ``workspace``: a
     Workspace the call uses instead of the library's per-stream one."""
-    import torch
     qs, qst = _shape4(q, "Q")
     ks, kst = _shape4(k, "K")
     vs, vst = _shape4(v, "V")
     _require_f32_cuda(q, k, v)
     if out is None:
-        out = torch.empty(tuple(qs), dtype=torch.float32, device=q.device)
-    wsp, keep = None, None
+        out = q.new_empty(qs)
+    wsp = None
     if workspace is not None and qs[1] == ks[1]:
-        wsp, keep = _ws_arg(workspace, attention_workspace_size(qs, ks, is_causal), stream)
-    check(lib().nne_flash_attention_forward_ws(
-        q.data_ptr(), _i64(qs), _i64(qst), k.data_ptr(), _i64(ks), _i64(kst),
-        v.data_ptr(), _i64(vs), _i64(vst), out.data_ptr(), _i64(out.stride()),
-        int(bool(is_causal)), int(scale is not None), float(scale or 0.0),
+        wsp = _ws_arg(workspace, attention_workspace_size(qs, ks, is_causal), stream)
+    check(_native().flash(
+        q.data_ptr(), qs, qst, k.data_ptr(), ks, kst, v.data_ptr(), vs, vst,
+        out.data_ptr(), out.stride(), bool(is_causal), scale is not None, float(scale or 0.0),
         int(block_size_r), int(block_size_c), wsp, _stream(stream)))
     return out
 
@@ -292,22 +335,19 @@ def attention_forward(q, k, v, is_causal, q_offset=0, scale=None, out=None, stre
     with is_causal, key c is visible to row r iff c <= r + q_offset.
     ``workspace``: a Workspace the call uses instead of the library's
     per-stream one."""
-    import torch
     qs, qst = _shape4(q, "Q")
     ks, kst = _shape4(k, "K")
     vs, vst = _shape4(v, "V")
     _require_f32_cuda(q, k, v)
     if out is None:
-        out = torch.empty(tuple(qs), dtype=torch.float32, device=q.device)
-    wsp, keep = None, None
+        out = q.new_empty(qs)
+    wsp = None
     if workspace is not None:
-        wsp, keep = _ws_arg(workspace, attention_workspace_size(qs, ks, is_causal, q_offset),
-                            stream)
-    check(lib().nne_attention_forward_ws(
-        q.data_ptr(), _i64(qs), _i64(qst), k.data_ptr(), _i64(ks), _i64(kst),
-        v.data_ptr(), _i64(vs), _i64(vst), out.data_ptr(), _i64(out.stride()),
-        int(bool(is_causal)), int(q_offset), int(scale is not None), float(scale or 0.0),
-        wsp, _stream(stream)))
+        wsp = _ws_arg(workspace, attention_workspace_size(qs, ks, is_causal, q_offset), stream)
+    check(_native().attention(
+        q.data_ptr(), qs, qst, k.data_ptr(), ks, kst, v.data_ptr(), vs, vst,
+        out.data_ptr(), out.stride(), bool(is_causal), int(q_offset), scale is not None,
+        float(scale or 0.0), wsp, _stream(stream)))
     return out
 
 
@@ -388,6 +428,7 @@ class KVCache:
                          for _ in range(num_layers)]
         self.lens_host = [np.zeros(self.batch, dtype=np.int32) for _ in range(num_layers)]
         self._ws = Workspace(device) if own_workspace else None
+        self._decode_sizes = {}     # geometry -> NneWorkspaceSize, None where no decode call takes it
         self._engaged = [False] * num_layers    # Some(..) in the reference's slot vector
 
     @property
@@ -439,7 +480,7 @@ class KVCache:
         lh = self.lens_host[layer_idx]
         check(lib().nne_kv_append(
             self.k[layer_idx].data_ptr(), self.v[layer_idx].data_ptr(),
-            self.lens_dev[layer_idx].data_ptr(), lh.ctypes.data_as(_i32p),
+            self.lens_dev[layer_idx].data_ptr(), lh.ctypes.data,
             k_new.data_ptr(), _i64(k_new.stride()), v_new.data_ptr(), _i64(v_new.stride()),
             self.batch, self.num_kv_heads, self.capacity, self.head_dim, t, _stream(stream)))
         self._engaged[layer_idx] = True
@@ -452,29 +493,38 @@ class KVCache:
         keep-alive).  The library allocates nothing for these calls."""
         if self._ws is None:
             return None, None      # the library's per-stream workspace
-        size = NneWorkspaceSize()
-        rc = lib().nne_decode_workspace_size(self.batch, num_heads, self.num_kv_heads,
-                                             self.head_dim, ctypes.byref(size))
-        if rc != NNE_OK:
+        size = self._decode_size(num_heads)
+        if size is None:
             return None, None      # the call itself reports the geometry error
         self._ws.reserve(size, stream)
         return self._ws.struct()
 
+    def _decode_ws(self, num_heads, stream):
+        """workspace(), as the native calls take it."""
+        size = self._decode_size(num_heads) if self._ws is not None else None
+        return None if size is None else _ws_arg(self._ws, size, stream)
+
+    def _decode_size(self, num_heads):
+        key = (self.batch, num_heads, self.num_kv_heads, self.head_dim)
+        if key not in self._decode_sizes:
+            size = NneWorkspaceSize()
+            ok = lib().nne_decode_workspace_size(max(key[0], 1), *key[1:],
+                                                 ctypes.byref(size)) == NNE_OK
+            self._decode_sizes[key] = size if ok else None
+        return self._decode_sizes[key]
+
     def attend(self, layer_idx, q, out=None, scale=None, stream=None):
         """Decode attention of q [B, Hq, 1, d] over the cached rows."""
-        import torch
         self._check_layer(layer_idx)
         _require_f32_cuda(q)
         hq = q.shape[1]
         if out is None:
-            out = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-        wsp, keep = self.workspace(hq, stream)
-        check(lib().nne_decode_attention(
-            q.data_ptr(), _i64(q.stride()), self.k[layer_idx].data_ptr(),
-            self.v[layer_idx].data_ptr(), self.lens_dev[layer_idx].data_ptr(),
-            self.lens_host[layer_idx].ctypes.data_as(_i32p), out.data_ptr(), _i64(out.stride()),
-            self.batch, hq, self.num_kv_heads, self.capacity, self.head_dim,
-            int(scale is not None), float(scale or 0.0), wsp, _stream(stream)))
+            out = q.new_empty(q.shape)
+        check(_native().decode_attention(
+            q.data_ptr(), q.stride(), self.k[layer_idx].data_ptr(), self.v[layer_idx].data_ptr(),
+            self.lens_dev[layer_idx].data_ptr(), self.lens_host[layer_idx], out.data_ptr(),
+            out.stride(), self.batch, hq, self.num_kv_heads, self.capacity, self.head_dim,
+            scale is not None, float(scale or 0.0), self._decode_ws(hq, stream), _stream(stream)))
         return out
 
     def decode_step(self, layer_idx, q, k_new, v_new, out=None, scale=None, stream=None):
@@ -484,22 +534,19 @@ class KVCache:
         sequences' lengths.  Geometries the fused decode kernel does not take
         (a head dim that is not a multiple of 4) append with the append kernel
         and attend with the attention kernel, one call per distinct length."""
-        import torch
         self._check_layer(layer_idx)
         _require_f32_cuda(q, k_new, v_new)
         hq = q.shape[1]
         if out is None:
-            out = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-        if not decode_kernel_fits(self.batch, hq, self.num_kv_heads, self.head_dim):
+            out = q.new_empty(q.shape)
+        if self._decode_size(hq) is None:
             return self._append_then_attend(layer_idx, q, k_new, v_new, out, scale, stream)
-        wsp, keep = self.workspace(hq, stream)
-        check(lib().nne_decode_step(
-            q.data_ptr(), _i64(q.stride()), self.k[layer_idx].data_ptr(),
-            self.v[layer_idx].data_ptr(), self.lens_dev[layer_idx].data_ptr(),
-            self.lens_host[layer_idx].ctypes.data_as(_i32p), k_new.data_ptr(),
-            _i64(k_new.stride()), v_new.data_ptr(), _i64(v_new.stride()), out.data_ptr(),
-            _i64(out.stride()), self.batch, hq, self.num_kv_heads, self.capacity, self.head_dim,
-            int(scale is not None), float(scale or 0.0), wsp, _stream(stream)))
+        check(_native().decode_step(
+            q.data_ptr(), q.stride(), self.k[layer_idx].data_ptr(), self.v[layer_idx].data_ptr(),
+            self.lens_dev[layer_idx].data_ptr(), self.lens_host[layer_idx], k_new.data_ptr(),
+            k_new.stride(), v_new.data_ptr(), v_new.stride(), out.data_ptr(), out.stride(),
+            self.batch, hq, self.num_kv_heads, self.capacity, self.head_dim,
+            scale is not None, float(scale or 0.0), self._decode_ws(hq, stream), _stream(stream)))
         self._engaged[layer_idx] = True
         return out
 
@@ -616,7 +663,7 @@ class RotaryEmbedding:
         check(lib().nne_rope_apply(
             x.data_ptr(), _i64(x.shape), _i64(x.stride()), out.data_ptr(), _i64(out.stride()),
             self.cos.data_ptr(), self.sin.data_ptr(), self.max_seq_len, self.head_dim,
-            sp_d.data_ptr(), sp_h.ctypes.data_as(_i32p), _stream(stream)))
+            sp_d.data_ptr(), sp_h.ctypes.data, _stream(stream)))
         return out
 
 
@@ -647,18 +694,16 @@ def qkv_rope(x, w_packed, bq, bk, bv, rope, pos_dev, pos_host, num_heads, num_kv
     (the MultiHeadAttention projections) and ``head_dim`` gives d.
     ``workspace``: a Workspace the call uses instead of the library's
     per-stream one."""
-    import torch
     x2 = x.reshape(x.shape[0], x.shape[-1]) if x.dim() == 3 else x
     _require_f32_cuda(x2, w_packed)
     b, c = x2.shape
     d = rope.head_dim if rope is not None else int(head_dim)
-    dev = x2.device
     if q_out is None:
-        q_out = torch.empty((b, num_heads, 1, d), dtype=torch.float32, device=dev)
+        q_out = x2.new_empty((b, num_heads, 1, d))
     if k_out is None:
-        k_out = torch.empty((b, num_kv_heads, 1, d), dtype=torch.float32, device=dev)
+        k_out = x2.new_empty((b, num_kv_heads, 1, d))
     if v_out is None:
-        v_out = torch.empty((b, num_kv_heads, 1, d), dtype=torch.float32, device=dev)
+        v_out = x2.new_empty((b, num_kv_heads, 1, d))
     def ptr(t):
         return None if t is None else t.data_ptr()
 
@@ -668,15 +713,15 @@ def qkv_rope(x, w_packed, bq, bk, bv, rope, pos_dev, pos_host, num_heads, num_kv
     if rope is not None:
         pos_host = np.ascontiguousarray(pos_host, dtype=np.int32)
         tables = (rope.cos.data_ptr(), rope.sin.data_ptr(), rope.max_seq_len, rope.head_dim,
-                  pos_dev.data_ptr(), pos_host.ctypes.data_as(_i32p))
+                  pos_dev.data_ptr(), pos_host)
     else:
         tables = (None, None, 0, d, None, None)
-    wsp, keep = None, None
+    wsp = None
     if workspace is not None:
         size = NneWorkspaceSize()
         check(lib().nne_qkv_workspace_size(c, num_heads, num_kv_heads, d, ctypes.byref(size)))
-        wsp, keep = _ws_arg(workspace, size, stream)
-    check(lib().nne_qkv_rope_ws(
+        wsp = _ws_arg(workspace, size, stream)
+    check(_native().qkv_rope(
         x2.data_ptr(), x2.stride(0), w_packed.data_ptr(), ptr(bq), ptr(bk), ptr(bv), *tables,
         q_out.data_ptr(), k_out.data_ptr(), v_out.data_ptr(), b, c, num_heads, num_kv_heads, d,
         wsp, _stream(stream)))

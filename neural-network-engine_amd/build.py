@@ -4,13 +4,15 @@
 
 produces neural-network-engine_amd/lib/libnne_attn.so (HIP kernels + C ABI) and
 neural-network-engine_amd/lib/libnne_host.so (the C++ host API of host/nne.hpp,
-on top of the C ABI and rocBLAS).
+on top of the C ABI and rocBLAS) and neural-network-engine_amd/lib/nne_pycall.so
+(the package's native call path).
 Every build recompiles; nothing is cached outside the repository, so the
 built file travels with the tree to the GPU machine.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -18,6 +20,7 @@ CSRC = os.path.join(PKG, "csrc")
 LIB_DIR = os.path.join(PKG, "lib")
 LIB = os.path.join(LIB_DIR, "libnne_attn.so")
 HOST_LIB = os.path.join(LIB_DIR, "libnne_host.so")
+CALL_LIB = os.path.join(LIB_DIR, "nne_pycall.so")
 
 SOURCES = ["prefill.hip", "small.hip", "splitk.hip", "splitk_plan.cpp", "qkv.hip", "deep.hip", "deep_plan.cpp", "abi.cpp", "noalloc.hip"]
 
@@ -47,7 +50,7 @@ def _run(cmd, out, verbose):
     noise = "is not a recognized feature for this target"
     err = "\n".join(l for l in res.stderr.splitlines() if noise not in l)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + err)
+        raise RuntimeError("%s failed:\n%s" % (cmd[0], err))
     if verbose and err.strip():
         print(err, file=sys.stderr)
     os.replace(tmp, out)
@@ -76,8 +79,17 @@ def build_host_library(verbose=False):
     return _run(cmd, HOST_LIB, verbose)
 
 
+def build_call_module(verbose=False):
+    """The CPython module that calls the C ABI (host code only)."""
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-I" + sysconfig.get_paths()["include"],
+           "-I" + os.path.join(ROOT, "include"),
+           os.path.join(CSRC, "pycall.cpp")]
+    return _run(cmd, CALL_LIB, verbose)
+
+
 def build_all(verbose=False):
-    return [build_library(verbose), build_host_library(verbose)]
+    return [build_library(verbose), build_host_library(verbose), build_call_module(verbose)]
 
 
 if __name__ == "__main__":
