@@ -177,15 +177,27 @@ int cut_chunks(const SplitKParams& p, int64_t x, int64_t ovh, int max_wg, int* e
     return count;
 }
 
-// The smallest budget whose cut fits `slots` workgroups (and at least 4
-// blocks and an eighth of the longest head, as for equal chunks).
+// The shortest chunk: a block for each of the 4 waves, an eighth of the longest
+// head while that is below 160 KB of K and V rows, then that, and 1/32 of it
+// past 5 MB.  Every part costs the merging workgroup a record (a head cut into
+// many short chunks waits longer for them than its keys take to stream), but a
+// long head on few workgroups streams at their rate alone.  Measured, one
+// sequence of 32 heads over 8 KV heads, d = 128, at 1/8, 1/16 and 1/32 of the
+// head: 8000 keys 28.4, 22.1, 19.2 us; 1733 keys 12.4, 13.6, 13.7 (12.4 at
+// 1/12); 16 heads over 2, 4000 keys 21.3, 18.1, 16.9; d = 64 cross-attention, 3000
+// keys 11.3, 11.6, 13.6.
+int64_t shortest_chunk(int d, int max_len) {
+    const int64_t eighth = (max_len + 7) / 8, rows = 160 * 128 / std::max(d, 1);
+    return std::max<int64_t>({4 * kKeyBlock, std::min(eighth, rows), (max_len + 31) / 32});
+}
+
+// The smallest budget whose cut fits `slots` workgroups.
 bool plan_cut(SplitKParams& p, int slots, int64_t total_keys, int max_len) {
     slots = std::min(slots, kMaxCutWg);
     if (!p.arg_pref_valid || !p.fused || total_keys == 0 || total_keys > INT32_MAX || slots < 1)
         return false;
     const int64_t ovh = cut_segment_keys(p.d);
-    int64_t lo = std::max<int64_t>((total_keys + slots - 1) / slots,
-                                   std::max<int64_t>(4 * kKeyBlock, (max_len + 7) / 8));
+    int64_t lo = std::max<int64_t>((total_keys + slots - 1) / slots, shortest_chunk(p.d, max_len));
     int64_t hi = lo;
     while (cut_chunks(p, hi, ovh, slots, nullptr) > slots) {
         if (hi > total_keys) return false;
@@ -206,11 +218,7 @@ bool plan_cut(SplitKParams& p, int slots, int64_t total_keys, int max_len) {
 void plan_equal(SplitKParams& p, int slots, int64_t total_keys, int max_len) {
     int64_t chunk = (total_keys + slots - 1) / (slots > 0 ? slots : 1);
     int64_t min_chunk = (max_len + (p.max_parts - 2) - 1) / (p.max_parts - 2);
-    if (min_chunk < 4 * kKeyBlock) min_chunk = 4 * kKeyBlock;   // a block for each of the 4 waves
-    // At most ~8 workgroups per head: a small problem (few, short heads)
-    // otherwise splits into many short chunks whose records cost the merging
-    // workgroup more round trips than the extra keys per chunk cost to stream.
-    if (min_chunk < (max_len + 7) / 8) min_chunk = (max_len + 7) / 8;
+    min_chunk = std::max(min_chunk, shortest_chunk(p.d, max_len));
     if (chunk < min_chunk) chunk = min_chunk;
     chunk = (chunk + kKeyBlock - 1) / kKeyBlock * kKeyBlock;
     if (chunk < kKeyBlock) chunk = kKeyBlock;
