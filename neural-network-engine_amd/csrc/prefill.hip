@@ -374,6 +374,10 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
     char* const Vs = lds + 3 * KP;
     char* const Qs = Vs + 3 * VP;
 
+    // Every argument's cache line in one round trip (left to the compiler, the
+    // first uses and the search below pay one each).
+    warm_kernargs<0, SPLIT ? sizeof(PrefillParams) : offsetof(PrefillParams, part_prefix)>();
+
     // ---- persistent workgroup: slot q of XCD x -------------------------------
     // Hardware dispatches consecutive workgroup ids round-robin over the 8
     // XCDs, so x = id & 7; each XCD owns a contiguous range of super-items
@@ -445,6 +449,28 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
         t1 = min(n_tiles, t0 + p.chunk_tiles);
     }
 
+    const float* kb = p.k.p + bi * p.k.sb + kvh * p.k.sh;
+    const float* vb = p.v.p + bi * p.v.sb + kvh * p.v.sh;
+
+    // The second item of a causal pair walks its key tiles backwards.  The
+    // workgroups of an XCD then stand at only two key positions at any time
+    // -- t on their first (long) items, total - t on their second (short)
+    // ones, whatever their ranks -- so the head's K/V tiles they read stay in
+    // the XCD's L2.  Walked forwards, every second item restarts at key 0 at
+    // its own time and the walks spread over the whole head: config 4 read
+    // 284 MB from HBM, 249 MB backwards (201 MB algorithmic); same time.
+    const bool rev = !SPLIT && p.pairing && (j & 1);
+    const int kstep = rev ? -1 : 1;
+    const int kfirst = rev ? t1 - 1 : t0;
+    const int n_it = t1 - t0;
+    Tile ld;
+    ld.init(p, wave, lane);
+    // The first tile's loads go before Q's, so that the two latencies overlap.
+    if (n_it > 0) {
+        ld.load_k(p, kb, kfirst * 32, wave, lane, true);
+        ld.load_v(p, vb, kfirst * 32, wave, lane, true);
+    }
+
     // ---- Q^T: three bf16 parts of Q[qrow][16t + 8*half + 0..7] * scale*log2(e)
     short8 qf[2][NT], ql[NT - NQL];
     char* const qls = Qs + (wave * NQL * 64 + lane) * 16;
@@ -484,9 +510,6 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
     }
     asm volatile("" : "+v"(q_code));   // computed here, not from every x after the loop
 
-    const float* kb = p.k.p + bi * p.k.sb + kvh * p.k.sh;
-    const float* vb = p.v.p + bi * p.v.sb + kvh * p.v.sh;
-
     floatx16 o[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -494,22 +517,7 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
         for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
     float m_run = kNegInf, l_run = 0.f;
 
-    // The second item of a causal pair walks its key tiles backwards.  The
-    // workgroups of an XCD then stand at only two key positions at any time
-    // -- t on their first (long) items, total - t on their second (short)
-    // ones, whatever their ranks -- so the head's K/V tiles they read stay in
-    // the XCD's L2.  Walked forwards, every second item restarts at key 0 at
-    // its own time and the walks spread over the whole head: config 4 read
-    // 284 MB from HBM, 249 MB backwards (201 MB algorithmic); same time.
-    const bool rev = !SPLIT && p.pairing && (j & 1);
-    const int kstep = rev ? -1 : 1;
-    const int kfirst = rev ? t1 - 1 : t0;
-    const int n_it = t1 - t0;
-    Tile ld;
-    ld.init(p, wave, lane);
     if (n_it > 0) {
-        ld.load_k(p, kb, kfirst * 32, wave, lane, true);
-        ld.load_v(p, vb, kfirst * 32, wave, lane, true);
         ld.store_k(Ks, wave, lane);
         ld.store_v(Vs, wave, lane);
     }
