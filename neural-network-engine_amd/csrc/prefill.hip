@@ -211,19 +211,22 @@ struct SplitTile {
         }
     }
 
+    // The parts of one load (4 dims of a key) computed and stored, for the
+    // caller to place between MFMAs; store_k does all NK.
+    __device__ __forceinline__ void part_k(int i, char* ks, int wave, int lane) const {
+        const int c4 = col_of(lane, i % NC) >> 2, c8 = c4 >> 1;   // 8-dim chunk 2t + h
+        const int r = KR * wave + row_of(lane) + RPI * (i / NC);
+        uint2 h, m, l;
+        split3(kr[i].x, kr[i].y, h.x, m.x, l.x);
+        split3(kr[i].z, kr[i].w, h.y, m.y, l.y);
+        char* a = ks + c8 * 512 + (c4 & 1) * 8 + ((r ^ (c8 & 15)) << 4);
+        *reinterpret_cast<uint2*>(a) = h;
+        *reinterpret_cast<uint2*>(a + K_PLANE) = m;
+        *reinterpret_cast<uint2*>(a + 2 * K_PLANE) = l;
+    }
     __device__ __forceinline__ void store_k(char* ks, int wave, int lane) const {
 #pragma unroll
-        for (int i = 0; i < NK; ++i) {
-            const int c4 = col_of(lane, i % NC) >> 2, c8 = c4 >> 1;   // 8-dim chunk 2t + h
-            const int r = KR * wave + row_of(lane) + RPI * (i / NC);
-            uint2 h, m, l;
-            split3(kr[i].x, kr[i].y, h.x, m.x, l.x);
-            split3(kr[i].z, kr[i].w, h.y, m.y, l.y);
-            char* a = ks + c8 * 512 + (c4 & 1) * 8 + ((r ^ (c8 & 15)) << 4);
-            *reinterpret_cast<uint2*>(a) = h;
-            *reinterpret_cast<uint2*>(a + K_PLANE) = m;
-            *reinterpret_cast<uint2*>(a + 2 * K_PLANE) = l;
-        }
+        for (int i = 0; i < NK; ++i) part_k(i, ks, wave, lane);
     }
 
     // Wave w reads the 8 keys of (step s, lane half h) = (w / 2 % 2, w % 2); with
@@ -263,21 +266,20 @@ struct SplitTile {
         }
     }
 
-    __device__ __forceinline__ void store_v(char* vs, int wave, int lane) const {
+    // Likewise two keys of a dim; every fourth step stores the dim's 8 keys.
+    uint32_t vp[3][4];
+    __device__ __forceinline__ void part_v(int i, char* vs, int wave, int lane) {
+        const int j = i >> 2, dim = dim_of(wave, lane, j);
+        split3(vr[j][2 * (i & 3)], vr[j][2 * (i & 3) + 1], vp[0][i & 3], vp[1][i & 3], vp[2][i & 3]);
+        if ((i & 3) != 3 || (64 * (j + 1) > VD && lane + 64 * j >= VD)) return;
+        char* a = vs + (((dim >> 5) * 2 + ((wave >> 1) & 1)) * 64 + (wave & 1) * 32 + (dim & 31)) * 16;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int dim = dim_of(wave, lane, j);
-            if (64 * (j + 1) > VD && lane + 64 * j >= VD) continue;
-            uint4 h, m, l;
-            split3(vr[j][0], vr[j][1], h.x, m.x, l.x);
-            split3(vr[j][2], vr[j][3], h.y, m.y, l.y);
-            split3(vr[j][4], vr[j][5], h.z, m.z, l.z);
-            split3(vr[j][6], vr[j][7], h.w, m.w, l.w);
-            char* a = vs + (((dim >> 5) * 2 + ((wave >> 1) & 1)) * 64 + (wave & 1) * 32 + (dim & 31)) * 16;
-            *reinterpret_cast<uint4*>(a) = h;
-            *reinterpret_cast<uint4*>(a + V_PLANE) = m;
-            *reinterpret_cast<uint4*>(a + 2 * V_PLANE) = l;
-        }
+        for (int u = 0; u < 3; ++u)
+            *reinterpret_cast<uint4*>(a + u * V_PLANE) = make_uint4(vp[u][0], vp[u][1], vp[u][2], vp[u][3]);
+    }
+    __device__ __forceinline__ void store_v(char* vs, int wave, int lane) {
+#pragma unroll
+        for (int i = 0; i < 4 * NJ; ++i) part_v(i, vs, wave, lane);
     }
 };
 
@@ -781,6 +783,16 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
 // phase apart as in the d <= 128 kernel (two barriers per tile); at 512 a tile
 // of either is 98 KB, so both go through one buffer (four barriers).  The low
 // parts of Q's last steps stay in LDS.
+//
+// What bounds it: the barriers.  The waves of a CU run their MFMAs and their
+// softmax at the same time; up to 256 dims the parts of K and V are therefore
+// computed between the MFMAs of the same wave (d = 256, T = 4096 820 -> 785 us,
+// d = 192 1830 -> 1690 us).  The matrix cores are busy 51 % of the cycles at 256
+// dims without that and 37 % at 512 (a staged tile serves only 64 rows there: 630
+// vector instructions beside 96 MFMAs per wave and tile).  Against the f32 MFMAs:
+// B = 1, H = 16, T = 4096 causal, d = 256 1190 -> 780 us, d = 512 2410 -> 1930 us;
+// B = 8, H = 20, T = 1500, d = 192 2570 -> 1690 us, at 0.6 to 0.7 of the error
+// against 64 bits.
 template <int DW, int NW, bool CAUSAL, bool VEC>
 __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParams p) {
     constexpr int D = DW * NW, U = 8 / NW;
@@ -885,7 +897,6 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
         ld.load_k(p, kb, kfirst * 32, wave, lane, true);
         ld.load_v(p, vb, kfirst * 32, wave, lane, true);
         ld.store_k(Ks, wave, lane);
-        if (!ONE) ld.store_v(Vs, wave, lane);
     }
     __syncthreads();
 
@@ -893,7 +904,6 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
         const int kt = kfirst + kstep * it;
         const bool has_next = it + 1 < n_tiles;
         const bool mine = kt < wave_tiles;
-        if (!ONE) ld.load_k(p, kb, (kt + kstep) * 32, wave, lane, has_next);
         floatx16 s;
         const float m_use = (m_run == kNegInf) ? 0.f : m_run;
         if (mine) {
@@ -902,41 +912,43 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
             for (int r = 0; r < 16; ++r) s[r] = 0.f;
             const char* kw = Ks + dq * NT * 1024;
             __builtin_amdgcn_s_setprio(1);
+            // The operands of a step are read one step ahead; between the later
+            // steps (its loads are still under way before) this tile's V is
+            // split, which no other wave of the SIMD would hide: all of a
+            // workgroup's waves run their MFMAs at the same time.
+            short8 kc[3], kn[3];
+            const auto read_k = [&](int t, short8* f) {
+                const char* a = kw + t * 1024 + half * 512 + ((l32 ^ ((2 * (dq * NT + t) + half) & 15)) << 4);
+                f[0] = *reinterpret_cast<const short8*>(a);
+                f[1] = *reinterpret_cast<const short8*>(a + KP);
+                f[2] = *reinterpret_cast<const short8*>(a + 2 * KP);
+            };
+            read_k(0, kc);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const char* a = kw + t * 1024 + half * 512 + ((l32 ^ ((2 * (dq * NT + t) + half) & 15)) << 4);
-                const short8 kh = *reinterpret_cast<const short8*>(a);
-                const short8 km = *reinterpret_cast<const short8*>(a + KP);
-                const short8 kl = *reinterpret_cast<const short8*>(a + 2 * KP);
-                s = mfma_bf16(kl, qf[0][t], s);
-                s = mfma_bf16(kh, t < NT - NQL ? ql[t < NT - NQL ? t : 0]
-                                               : *reinterpret_cast<const short8*>(
-                                                     qls + (t - (NT - NQL)) * 1024), s);
-                s = mfma_bf16(km, qf[1][t], s);
-                s = mfma_bf16(km, qf[0][t], s);
-                s = mfma_bf16(kh, qf[1][t], s);
+                short8 qlt;
+                if (t < NT - NQL) qlt = ql[t < NT - NQL ? t : 0];
+                else qlt = *reinterpret_cast<const short8*>(qls + (t - (NT - NQL)) * 1024);
+                if (t + 1 < NT) read_k(t + 1, kn);
+                s = mfma_bf16(kc[2], qf[0][t], s);
+                s = mfma_bf16(kc[1], qf[1][t], s);
+                s = mfma_bf16(kc[1], qf[0][t], s);
+                s = mfma_bf16(kc[0], qf[1][t], s);
+                s = mfma_bf16(kc[0], qlt, s);
+                if (!ONE) {
+#pragma unroll
+                    for (int i = 0; i < 4 * Tile::NJ; ++i)
+                        if (NT / 2 + i * (NT / 2) / (4 * Tile::NJ) == t) ld.part_v(i, Vs, wave, lane);
+                }
+#pragma unroll
+                for (int u = 0; u < 3; ++u) kc[u] = kn[u];
+                __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 const char* a = kw + t * 1024 + half * 512 + ((l32 ^ ((2 * (dq * NT + t) + half) & 15)) << 4);
                 s = mfma_bf16(*reinterpret_cast<const short8*>(a), qf[0][t], s);
             }
-            // Schedule: the operands of a step are read one step ahead.
-            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-#pragma unroll
-            for (int t = 0; t < NT - 1; ++t) {
-                if (t + 1 < NT - NQL) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-                else __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 5, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 5, 0);
-#pragma unroll
-            for (int t = 0; t < NT - 2; ++t) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
             __builtin_amdgcn_s_setprio(0);
             // This wave's partial, register-group major (each store one
             // contiguous, conflict-free 1 KB wave access).
@@ -945,14 +957,14 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
             for (int i = 0; i < 4; ++i)
                 *reinterpret_cast<float4*>(xo + 1024 * i) =
                     make_float4(s[4 * i], s[4 * i + 1], s[4 * i + 2], s[4 * i + 3]);
+        } else if (!ONE) {
+            ld.store_v(Vs, wave, lane);
         }
+        if (!ONE) ld.load_k(p, kb, (kt + kstep) * 32, wave, lane, has_next);
         __syncthreads();   // partials visible, K read (and V visible)
         if (ONE) {
             ld.store_v(Vs, wave, lane);
             ld.load_k(p, kb, (kt + kstep) * 32, wave, lane, has_next);
-        } else {
-            if (has_next) ld.store_k(Ks, wave, lane);
-            ld.load_v(p, vb, (kt + kstep) * 32, wave, lane, has_next);
         }
         if (mine) {
             // S^T - m: the unit's partials in wave order.
@@ -1007,47 +1019,63 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
         }
         if (ONE) __syncthreads();   // V visible
         if (mine) {
-            // O^T += V^T P^T over this wave's output dims.
+            // O^T += V^T P^T over this wave's output dims, the next K split
+            // between the MFMAs.
+            uint32_t pp[2][3][4];
+            const auto part_p = [&](int i) {
+                split3(s[2 * i], s[2 * i + 1], pp[i >> 2][0][i & 3], pp[i >> 2][1][i & 3], pp[i >> 2][2][i & 3]);
+            };
+            const auto operand = [&](int st, int u) {
+                return __builtin_bit_cast(short8, make_uint4(pp[st][u][0], pp[st][u][1], pp[st][u][2], pp[st][u][3]));
+            };
+            short8 vc[3], vn[3];
+            const auto read_v = [&](int i, short8* f) {
+                const char* a = Vs + (((dq * NB + i % NB) * 2 + i / NB) * 64 + lane) * 16;
+                f[0] = *reinterpret_cast<const short8*>(a);
+                f[1] = *reinterpret_cast<const short8*>(a + KP);
+                f[2] = *reinterpret_cast<const short8*>(a + 2 * KP);
+            };
+            if (!ONE) read_v(0, vc);   // (read ahead: 12 registers that 512 dims do not have)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part_p(i);
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                uint4 h, m, l;
-                split3(s[8 * st + 0], s[8 * st + 1], h.x, m.x, l.x);
-                split3(s[8 * st + 2], s[8 * st + 3], h.y, m.y, l.y);
-                split3(s[8 * st + 4], s[8 * st + 5], h.z, m.z, l.z);
-                split3(s[8 * st + 6], s[8 * st + 7], h.w, m.w, l.w);
-                const short8 ph = __builtin_bit_cast(short8, h), pm = __builtin_bit_cast(short8, m),
-                             pl = __builtin_bit_cast(short8, l);
+            for (int i = 0; i < 2 * NB; ++i) {
+                const int b = i % NB, st = i / NB;
+                if (ONE) read_v(i, vc);
+                else if (i + 1 < 2 * NB) read_v(i + 1, vn);
+                const short8 ph = operand(st, 0), pm = operand(st, 1), pl = operand(st, 2);
+                o[b] = mfma_bf16(vc[2], ph, o[b]);
+                o[b] = mfma_bf16(vc[0], pl, o[b]);
+                o[b] = mfma_bf16(vc[1], pm, o[b]);
+                o[b] = mfma_bf16(vc[1], ph, o[b]);
+                o[b] = mfma_bf16(vc[0], pm, o[b]);
+                o[b] = mfma_bf16(vc[0], ph, o[b]);
+                if (st == 0) {
 #pragma unroll
-                for (int b = 0; b < NB; ++b) {
-                    const char* a = Vs + (((dq * NB + b) * 2 + st) * 64 + lane) * 16;
-                    const short8 vh = *reinterpret_cast<const short8*>(a);
-                    const short8 vm = *reinterpret_cast<const short8*>(a + KP);
-                    const short8 vl = *reinterpret_cast<const short8*>(a + 2 * KP);
-                    o[b] = mfma_bf16(vl, ph, o[b]);
-                    o[b] = mfma_bf16(vh, pl, o[b]);
-                    o[b] = mfma_bf16(vm, pm, o[b]);
-                    o[b] = mfma_bf16(vm, ph, o[b]);
-                    o[b] = mfma_bf16(vh, pm, o[b]);
-                    o[b] = mfma_bf16(vh, ph, o[b]);
+                    for (int u = 4 + 4 * b / NB; u < 4 + 4 * (b + 1) / NB; ++u) part_p(u);
                 }
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                if (!ONE) {
 #pragma unroll
-            for (int i = 0; i < 2 * NB - 1; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+                    for (int u = i * Tile::NK / (2 * NB); u < (i + 1) * Tile::NK / (2 * NB); ++u)
+                        ld.part_k(u, Ks, wave, lane);
+                }
+                if (!ONE) {
+#pragma unroll
+                    for (int u = 0; u < 3; ++u) vc[u] = vn[u];
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
             __builtin_amdgcn_s_setprio(0);
+        } else if (!ONE) {
+            ld.store_k(Ks, wave, lane);
         }
+        if (!ONE) ld.load_v(p, vb, (kt + kstep) * 32, wave, lane, has_next);
         __syncthreads();   // V and the partials are read (and the next K visible)
         if (ONE) {
             if (has_next) ld.store_k(Ks, wave, lane);
             ld.load_v(p, vb, (kt + kstep) * 32, wave, lane, has_next);
             __syncthreads();   // the next K is visible
-        } else {
-            if (has_next) ld.store_v(Vs, wave, lane);
         }
     }
 
