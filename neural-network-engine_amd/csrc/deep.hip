@@ -1,6 +1,7 @@
 // Attention at head dims above 256: prefill, cross-attention and decode over a
-// KV cache, on v_mfma_f32_32x32x2_f32; and prefill at 129-256 dims that the
-// wave-pair kernel does not take (dims other than 256, small problems).
+// KV cache, on v_mfma_f32_32x32x2_f32; and prefill at 129-256 dims.  Prefill up
+// to 512 dims with more 32-row units than CUs (above 256 dims, causal: than two
+// per CU) runs on prefill_wide_kernel instead, on the bf16 matrix cores.
 //
 // Algorithm: the online softmax of the reference's flash_attention_forward
 // (src/nn/flash_attention.rs:91-195) over 32-key tiles, rows that see no key
@@ -34,7 +35,9 @@
 //    per half-wave.
 //  * The next tile's K (up to 8 chunks) is loaded during the current tile's
 //    exchange, softmax and P V, and a tile's V at its start, under its S.
-//  Prefill problems with more workgroups than CUs use a 4-wave form
+//  Up to 512 dims, full units on more workgroups than CUs (those that
+//  prefill_wide_kernel does not take: decode steps of 32 query heads or more
+//  per KV head, K/V row strides beyond that kernel's) use a 4-wave form
 //  instead, two workgroups per CU: each wave takes twice the chunks and
 //  output blocks (S from 4 partials, Q^T of its last 8 chunks in LDS), so a
 //  tile's MFMAs per wave double against the same exchange and softmax, and
@@ -600,7 +603,7 @@ hipError_t launch_deep_v(DeepParams p, hipStream_t stream) {
 // long one runs alone with one wave per SIMD), and so do decode steps (a few
 // rows per unit, streaming their caches: B = 32, d = 512 634 us with 8
 // waves, 781 us with 4).
-// Head dims 129-256 (prefill the wave-pair kernel does not take) run the
+// Head dims 129-256 (prefill with at most as many 32-row units as CUs) run the
 // 2-wave form unsplit, and the 8-wave form's key split.
 template <bool CAUSAL>
 hipError_t launch_deep_t(const DeepParams& p, int cus, hipStream_t stream) {
