@@ -52,9 +52,12 @@ __device__ __forceinline__ floatx16 mfma_bf16(short8 a, short8 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
+// The conversions and the MFMAs keep bf16's subnormals, so the parts hold a value
+// down to 2^-133, whole from 2^-110 up.  Softmax weights come as small as 2^-126
+// and are split 2^16 times their size (a weight of 2^-124 on a V beyond 2^100
+// times the others' is a result like any other: without it 3e-4 of error there).
 // Where the parts do not hold a value: an infinity, a NaN or a magnitude that
-// rounds to infinity leaves NaN parts, and every result it enters is NaN; below
-// 2^-100 the low parts fall under bf16's normal range, which the MFMAs flush.
+// rounds to infinity leaves NaN parts, and every result it enters is NaN.
 // Results show both (a tiny V gives tiny O), except where a tiny query meets a
 // huge key or a huge query a tiny key, so queries have a range of their own.
 // (range_code: 0 for zero, ascending with the magnitude from 2^-90 on, above
@@ -63,6 +66,7 @@ __device__ __forceinline__ uint32_t range_code(float x) {
     const uint32_t a = __float_as_uint(x) & 0x7fffffffu;
     return a == 0 ? 0 : a - __float_as_uint(0x1p-90f);
 }
+constexpr float kPartUp = 0x1p16f, kPartDown = 0x1p-16f;
 constexpr uint32_t kResultCodes = 0x7f800000u - 0x12800000u;   // codes of finite results
 constexpr uint32_t kQueryCodes = 0x6c800000u - 0x12800000u;    // codes of queries up to 2^90
 

@@ -630,10 +630,10 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
                 uint4 h, m, l;
-                split3(s[8 * st + 0], s[8 * st + 1], h.x, m.x, l.x);
-                split3(s[8 * st + 2], s[8 * st + 3], h.y, m.y, l.y);
-                split3(s[8 * st + 4], s[8 * st + 5], h.z, m.z, l.z);
-                split3(s[8 * st + 6], s[8 * st + 7], h.w, m.w, l.w);
+                split3(s[8 * st + 0] * kPartUp, s[8 * st + 1] * kPartUp, h.x, m.x, l.x);
+                split3(s[8 * st + 2] * kPartUp, s[8 * st + 3] * kPartUp, h.y, m.y, l.y);
+                split3(s[8 * st + 4] * kPartUp, s[8 * st + 5] * kPartUp, h.z, m.z, l.z);
+                split3(s[8 * st + 6] * kPartUp, s[8 * st + 7] * kPartUp, h.w, m.w, l.w);
                 const short8 ph = __builtin_bit_cast(short8, h), pm = __builtin_bit_cast(short8, m),
                              pl = __builtin_bit_cast(short8, l);
 #pragma unroll
@@ -670,8 +670,11 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
     for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o_code = max(o_code, range_code(o[b][r]));
-    if (__builtin_amdgcn_ballot_w64(q_code > kQueryCodes || o_code >= kResultCodes) != 0)
+    float down = kPartDown;   // what a result is to be multiplied with
+    if (__builtin_amdgcn_ballot_w64(q_code > kQueryCodes || o_code >= kResultCodes) != 0) {
         unit_f32<D, NB, CAUSAL>(p, head, unit, t0, min(t1, wave_tiles), 0, o, m_run, l_run);
+        down = 1.f;
+    }
 
     float l_tot = pair_sum(l_run);
     if constexpr (SPLIT) {
@@ -687,7 +690,7 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) store_coherent(wo + (b * 16 + r) * 64, o[b][r]);
+                    for (int r = 0; r < 16; ++r) store_coherent(wo + (b * 16 + r) * 64, o[b][r] * down);
                 float* wml = p.ws + (((int64_t)pair * 4 + wave) * 64 + lane) * 2;
                 store_coherent(wml, m_run);
                 store_coherent(wml + 1, l_tot);
@@ -708,6 +711,7 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
             constexpr int GRP = D >= 128 ? 2 : 4;
             float M = kNegInf;
             l_tot = 0.f;
+            down = 1.f;
 #pragma unroll
             for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -745,7 +749,7 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
     }
 
     // ---- normalise and write O[qrow][dim], dim = 32b + 8(r/4) + 4*half + r%4 --
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    const float inv = l_tot > 0.f ? down / l_tot : 0.f;
     if (active && qrow < p.Tq) {
         float* op = p.o.p + bi * p.o.sb + hq * p.o.sh + (int64_t)qrow * p.o.st;
 #pragma unroll
@@ -1023,7 +1027,8 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
             // between the MFMAs.
             uint32_t pp[2][3][4];
             const auto part_p = [&](int i) {
-                split3(s[2 * i], s[2 * i + 1], pp[i >> 2][0][i & 3], pp[i >> 2][1][i & 3], pp[i >> 2][2][i & 3]);
+                split3(s[2 * i] * kPartUp, s[2 * i + 1] * kPartUp, pp[i >> 2][0][i & 3], pp[i >> 2][1][i & 3],
+                       pp[i >> 2][2][i & 3]);
             };
             const auto operand = [&](int st, int u) {
                 return __builtin_bit_cast(short8, make_uint4(pp[st][u][0], pp[st][u][1], pp[st][u][2], pp[st][u][3]));
@@ -1084,11 +1089,14 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
     for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o_code = max(o_code, range_code(o[b][r]));
-    if (__builtin_amdgcn_ballot_w64(o_code >= kResultCodes) != 0)
+    float down = kPartDown;
+    if (__builtin_amdgcn_ballot_w64(o_code >= kResultCodes) != 0) {
         unit_f32<D, NB, CAUSAL>(p, head, unit, 0, wave_tiles, dq * DW, o, m_run, l_run);
+        down = 1.f;
+    }
 
     const float l_tot = pair_sum(l_run);
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    const float inv = l_tot > 0.f ? down / l_tot : 0.f;
     if (active && qrow < p.Tq) {
         float* op = p.o.p + bi * p.o.sb + hq * p.o.sh + (int64_t)qrow * p.o.st;
 #pragma unroll

@@ -142,3 +142,26 @@ def test_row_strides_beyond_the_vector_loads():
     o = nne.attention_forward(torch.from_numpy(q).cuda(), kd, vd, False)
     torch.cuda.synchronize()
     check64(o.cpu().numpy(), attend64(q, k, v, False))
+
+
+@pytest.mark.parametrize("b", [1, 4])       # the key split and the unsplit launch
+@pytest.mark.parametrize("d", [20, 64, 128, 192, 256, 512])
+@pytest.mark.parametrize("bits", [112, 124])
+def test_tiny_weights_keep_their_bits(b, d, bits):
+    """Key 0 takes nearly all of the weight with a V of zeros; every other key's
+    weight is about 2^-bits on V of 2^60.  The scores share their roundings, each
+    at most 2^-24 of `bits`: of the scale, its log2 form, the query times it, two
+    in the sum and the difference from the maximum; times ln 2 that is the error."""
+    t = 300 if d <= 128 else 97
+    h = 40 if d <= 128 else 140 // b
+    q, k, v = draw(d + bits, b, h, h, t, t, d)
+    q[..., 1:] *= np.float32(0.05)
+    k[..., 1:] *= np.float32(0.05)
+    q[..., 0] = 1
+    k[..., 0] = -bits * np.log(2) * np.sqrt(d)
+    k[..., 0, 0] = 0
+    v *= np.float32(2.0**60)
+    v[..., 0, :] = 0
+    ref = attend64(q, k, v, False)
+    o = run(q, k, v, False)
+    assert np.linalg.norm(o - ref) <= 6 * bits * 2.0**-24 * np.log(2) * np.linalg.norm(ref)
