@@ -55,19 +55,20 @@ __device__ __forceinline__ floatx16 mfma_bf16(short8 a, short8 b, floatx16 c) {
 // The conversions and the MFMAs keep bf16's subnormals, so the parts hold a value
 // down to 2^-133, whole from 2^-110 up.  Softmax weights come as small as 2^-126
 // and are split 2^16 times their size (a weight of 2^-124 on a V beyond 2^100
-// times the others' is a result like any other: without it 3e-4 of error there).
+// times the others' is a result like any other: without it 3e-4 of error there),
+// and so is V, whose parts are then whole at any size (subnormals are multiples
+// of 2^-133; unscaled, a V of 1e-42 gave zeros).
 // Where the parts do not hold a value: an infinity, a NaN or a magnitude that
-// rounds to infinity leaves NaN parts, and every result it enters is NaN.
-// Results show both (a tiny V gives tiny O), except where a tiny query meets a
-// huge key or a huge query a tiny key, so queries have a range of their own.
+// rounds or grows to infinity leaves NaN parts, and every result it enters is not
+// finite.  A tiny query that meets a huge key, or a huge query that meets a tiny
+// key, does not show there, so queries have a range of their own.
 // (range_code: 0 for zero, ascending with the magnitude from 2^-90 on, above
 // every such code for smaller magnitudes.)
 __device__ __forceinline__ uint32_t range_code(float x) {
     const uint32_t a = __float_as_uint(x) & 0x7fffffffu;
     return a == 0 ? 0 : a - __float_as_uint(0x1p-90f);
 }
-constexpr float kPartUp = 0x1p16f, kPartDown = 0x1p-16f;
-constexpr uint32_t kResultCodes = 0x7f800000u - 0x12800000u;   // codes of finite results
+constexpr float kPartUp = 0x1p16f, kPartDown = 0x1p-32f;   // of a weight or value, of their product
 constexpr uint32_t kQueryCodes = 0x6c800000u - 0x12800000u;    // codes of queries up to 2^90
 
 // Brings [B0, E0) and [B1, E1) of the kernel argument block into the scalar

@@ -270,7 +270,8 @@ struct SplitTile {
     uint32_t vp[3][4];
     __device__ __forceinline__ void part_v(int i, char* vs, int wave, int lane) {
         const int j = i >> 2, dim = dim_of(wave, lane, j);
-        split3(vr[j][2 * (i & 3)], vr[j][2 * (i & 3) + 1], vp[0][i & 3], vp[1][i & 3], vp[2][i & 3]);
+        split3(vr[j][2 * (i & 3)] * kPartUp, vr[j][2 * (i & 3) + 1] * kPartUp, vp[0][i & 3], vp[1][i & 3],
+               vp[2][i & 3]);
         if ((i & 3) != 3 || (64 * (j + 1) > VD && lane + 64 * j >= VD)) return;
         char* a = vs + (((dim >> 5) * 2 + ((wave >> 1) & 1)) * 64 + (wave & 1) * 32 + (dim & 31)) * 16;
 #pragma unroll
@@ -282,6 +283,16 @@ struct SplitTile {
         for (int i = 0; i < 4 * NJ; ++i) part_v(i, vs, wave, lane);
     }
 };
+
+template <int NB>
+__device__ __forceinline__ bool finite(const floatx16 (&o)[NB]) {
+    uint32_t most = 0;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) most = max(most, __float_as_uint(o[b][r]) & 0x7fffffffu);
+    return most < 0x7f800000u;
+}
 
 // One 32-row unit (its output dims dim0 .. dim0 + 32 NB - 1) over key tiles
 // [t0, t1) in plain f32 MFMAs on operands read from global memory: the arithmetic for inputs outside the range in which the
@@ -665,13 +676,8 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
 
     // Inputs the bf16 parts do not hold show in the result; such a unit is
     // computed again in f32.
-    uint32_t o_code = 0;
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o_code = max(o_code, range_code(o[b][r]));
     float down = kPartDown;   // what a result is to be multiplied with
-    if (__builtin_amdgcn_ballot_w64(q_code > kQueryCodes || o_code >= kResultCodes) != 0) {
+    if (__builtin_amdgcn_ballot_w64(q_code > kQueryCodes || !finite(o)) != 0) {
         unit_f32<D, NB, CAUSAL>(p, head, unit, t0, min(t1, wave_tiles), 0, o, m_run, l_run);
         down = 1.f;
     }
@@ -1084,13 +1090,8 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
         }
     }
 
-    uint32_t o_code = 0;
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o_code = max(o_code, range_code(o[b][r]));
     float down = kPartDown;
-    if (__builtin_amdgcn_ballot_w64(o_code >= kResultCodes) != 0) {
+    if (__builtin_amdgcn_ballot_w64(!finite(o)) != 0) {
         unit_f32<D, NB, CAUSAL>(p, head, unit, 0, wave_tiles, dq * DW, o, m_run, l_run);
         down = 1.f;
     }

@@ -165,3 +165,17 @@ def test_tiny_weights_keep_their_bits(b, d, bits):
     ref = attend64(q, k, v, False)
     o = run(q, k, v, False)
     assert np.linalg.norm(o - ref) <= 6 * bits * 2.0**-24 * np.log(2) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("b", [1, 4])
+@pytest.mark.parametrize("d", [20, 64, 128, 192, 256, 512])
+@pytest.mark.parametrize("vs", [1e-35, 1e-39, 1e-42])
+def test_values_below_the_normal_range(b, d, vs):
+    """V and O down to the smallest subnormals, 2^-149 apart: one rounding there
+    and a few of 2^-24 of the value."""
+    t = 300 if d <= 128 else 97
+    h = 40 if d <= 128 else 140 // b
+    q, k, v = draw(d, b, h, h, t, t, d)
+    v *= np.float32(vs)
+    ref = attend64(q, k, v, True)
+    assert (np.abs(run(q, k, v, True) - ref) <= 2.0**-149 + 1e-5 * vs).all()
