@@ -179,3 +179,31 @@ def test_values_below_the_normal_range(b, d, vs):
     v *= np.float32(vs)
     ref = attend64(q, k, v, True)
     assert (np.abs(run(q, k, v, True) - ref) <= 2.0**-149 + 1e-5 * vs).all()
+
+
+@pytest.mark.parametrize("d", [32, 64, 128, 256, 512])
+def test_large_scores_keep_their_differences(d):
+    """Every score has 200 in common, spread over the dims.  In log2 units the
+    scores lie between 2^8 and 2^9, where one f32 rounding leaves 2^-15 / sqrt(12)
+    (root mean square) of a score and ln 2 times that, 6e-6, of a weight; the D/16
+    sums at growing sizes come to little more, 48 at full size to four times it."""
+    t, h = (300, 80) if d <= 128 else (97, 140)
+    q, k, v = draw(d, 1, h, h, t, t, d)
+    u = np.sign(np.random.default_rng(5).standard_normal(d)) * np.sqrt(200 / np.sqrt(d))
+    q, k = q + u.astype(np.float32), k + u.astype(np.float32)
+    ref = attend64(q, k, v, False)
+    assert np.linalg.norm(run(q, k, v, False) - ref) <= 8e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256, 512])
+def test_results_far_below_one_on_ordinary_values(d):
+    """Peaked scores over a V of ones and zeros: the results are the weights, down
+    to f32's smallest, each within 16 roundings of a score below 128 (2^-18 each,
+    times ln 2)."""
+    t, h = (300, 80) if d <= 128 else (97, 140)
+    q, k, _ = draw(d, 1, h, h, t, t, d)
+    q, k = q * np.float32(4), k * np.float32(4)
+    v = np.broadcast_to(np.eye(t, d, dtype=np.float32), (1, h, t, d)).copy()
+    ref = attend64(q, k, v, False)
+    seen = ref > 2.0**-124
+    assert (np.abs(run(q, k, v, False) - ref)[seen] <= 16 * 2.0**-18 * np.log(2) * ref[seen]).all()
