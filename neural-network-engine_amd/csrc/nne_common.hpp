@@ -62,14 +62,14 @@ __device__ __forceinline__ floatx16 mfma_bf16(short8 a, short8 b, floatx16 c) {
 // rounds or grows to infinity leaves NaN parts, and every result it enters is not
 // finite.  A tiny query that meets a huge key, or a huge query that meets a tiny
 // key, does not show there, so queries have a range of their own.
-// (range_code: 0 for zero, ascending with the magnitude from 2^-90 on, above
+// (range_code: 0 for zero, ascending with the magnitude from 2^-110 on, above
 // every such code for smaller magnitudes.)
 __device__ __forceinline__ uint32_t range_code(float x) {
     const uint32_t a = __float_as_uint(x) & 0x7fffffffu;
-    return a == 0 ? 0 : a - __float_as_uint(0x1p-90f);
+    return a == 0 ? 0 : a - __float_as_uint(0x1p-110f);
 }
 constexpr float kPartUp = 0x1p16f, kPartDown = 0x1p-32f;   // of a weight or value, of their product
-constexpr uint32_t kQueryCodes = 0x6c800000u - 0x12800000u;    // codes of queries up to 2^90
+constexpr uint32_t kQueryCodes = 0x6c800000u - 0x08800000u;    // codes of queries up to 2^90
 
 // Brings [B0, E0) and [B1, E1) of the kernel argument block into the scalar
 // cache: one load per 64-byte line, all issued before a single wait.  The

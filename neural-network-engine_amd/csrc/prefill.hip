@@ -295,13 +295,22 @@ __device__ __forceinline__ bool finite(const floatx16 (&o)[NB]) {
 }
 
 // One 32-row unit (its output dims dim0 .. dim0 + 32 NB - 1) over key tiles
-// [t0, t1) in plain f32 MFMAs on operands read from global memory: the arithmetic for inputs outside the range in which the
-// three bf16 parts hold all 24 bits.  Slow, and rare.  Everything it needs is
-// derived here from a few opaque scalars, so that nothing of it is computed
+// [t0, t1) in plain f32 MFMAs on operands read from global memory: the arithmetic
+// for inputs outside the range of the parts (infinities, NaN, magnitudes near the
+// top of f32's; scaled queries beyond 2^90 or below 2^-110).  Everything it needs
+// is derived here from a few opaque scalars, so that nothing of it is computed
 // ahead of, or kept in registers across, the main loop.
-template <int D, int NB, bool CAUSAL>
+//
+// What bounds it: its loads, 32 dims of K and Q or 4 keys of V at a time before 16
+// MFMAs or more.  With one NaN in every head's V, so that every unit comes here
+// after the bf16 products (us; without it; one dim pair and one key at a time;
+// all f32 from the start on K/V tiles in LDS): d = 64, B = 4, H = 20, T = 300 62 (26,
+// 108, 29); d = 128 108 (41, 216, 53); d = 256, H = 140, T = 97 95 (36, 213, 47);
+// d = 512 253 (81, 554, 82).
+template <int D, int NB, bool CAUSAL, bool VEC>
 __device__ __forceinline__ void unit_f32(const PrefillParams& p, int head, int unit, int t0, int t1,
                                          int dim0, floatx16 (&o)[NB], float& m_run, float& l_run) {
+    constexpr int NL = D == 32 ? 2 : 4;   // loads of K and Q at a time (32 dims: four workgroups per CU)
     int tid = threadIdx.x;
     float zero = 0.f;
     asm volatile("" : "+v"(tid), "+v"(zero), "+s"(head), "+s"(unit), "+s"(t0), "+s"(t1),
@@ -319,27 +328,50 @@ __device__ __forceinline__ void unit_f32(const PrefillParams& p, int head, int u
         for (int r = 0; r < 16; ++r) o[b][r] = zero;
     m_run = kNegInf;
     l_run = zero;
+    // Dims c .. c + 3 of a row (zeros past the last dim or row).
+    const auto load4 = [&](const float* row, int64_t sd, int c, bool ok) {
+        vf4 x = {0.f, 0.f, 0.f, 0.f};
+        if (VEC) {
+            if (ok && c < p.d) x = *reinterpret_cast<const vf4*>(row + c);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (ok && c + j < p.d) x[j] = row[(c + j) * sd];
+        }
+        return x;
+    };
 #pragma nounroll
     for (int kt = t0; kt < t1; ++kt) {
         const int key0 = kt * 32;
         const bool kok = key0 + l32 < p.Tk;
         const float* kp = kb + (int64_t)(kok ? key0 + l32 : 0) * p.k.st;
-        floatx16 s;
+        int c0 = 4 * half;
+        asm volatile("" : "+v"(c0));   // Q is read again each tile, not held across them
+        // Two sums per score: half the roundings in each.
+        floatx16 s, s2;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = zero;
+        for (int r = 0; r < 16; ++r) s[r] = s2[r] = zero;
 #pragma nounroll
-        for (int t = 0; t < D / 2; ++t) {
-            const int c = half * (D / 2) + t;
-            const float kx = kok && c < p.d ? kp[c * p.k.sd] : 0.f;
-            const float qx = rok && c < p.d ? qp[c * p.q.sd] * p.qscale : 0.f;
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kx, qx, s, 0, 0, 0);
+        for (int t = 0; t < D; t += 8 * NL) {
+            vf4 kx[NL], qx[NL];
+#pragma unroll
+            for (int i = 0; i < NL; ++i) kx[i] = load4(kp, p.k.sd, t + 8 * i + c0, kok);
+#pragma unroll
+            for (int i = 0; i < NL; ++i) qx[i] = load4(qp, p.q.sd, t + 8 * i + c0, rok);
+#pragma unroll
+            for (int i = 0; i < NL; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; j += 2) {
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[i][j], qx[i][j] * p.qscale, s, 0, 0, 0);
+                    s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[i][j + 1], qx[i][j + 1] * p.qscale, s2, 0, 0, 0);
+                }
         }
         float mt = kNegInf;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int key = key0 + 8 * (r >> 2) + 4 * half + (r & 3);
             const bool vis = key < p.Tk && (!CAUSAL || key <= qrow + p.q_offset);
-            s[r] = vis ? s[r] : kNegInf;
+            s[r] = vis ? s[r] + s2[r] : kNegInf;
             mt = fmaxf(mt, s[r]);
         }
         const float m_new = fmaxf(m_run, pair_max(mt));
@@ -351,21 +383,31 @@ __device__ __forceinline__ void unit_f32(const PrefillParams& p, int head, int u
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
         m_run = m_new;
-        int key = key0 + 4 * half;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float pr = fast_exp2(s[r] - m_use);
-            l_run += pr;
+        for (int g = 0; g < 4; ++g) {
+            // Four keys' V in registers at a time.
+            float vx[4][NB];
+            int key = key0 + 8 * g + 4 * half;
             asm volatile("" : "+v"(key));
-            const float* vp = vb + (int64_t)(key < p.Tk ? key : 0) * p.v.st;
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const int dim = dim0 + 32 * b + l32;
-                const float vx = key < p.Tk && dim < p.d ? vp[dim * p.v.sd] : 0.f;
-                o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx, pr, o[b], 0, 0, 0);
+            for (int j = 0; j < 4; ++j) {
+                const bool ok = key + j < p.Tk;
+                const float* vp = vb + (int64_t)(ok ? key + j : 0) * p.v.st;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const int dim = dim0 + 32 * b + l32;
+                    vx[j][b] = ok && dim < p.d ? vp[dim * p.v.sd] : 0.f;
+                }
             }
-            key += (r & 3) == 3 ? 5 : 1;
-            __builtin_amdgcn_sched_barrier(0);   // one key's V in registers at a time
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float pr = fast_exp2(s[4 * g + j] - m_use);
+                l_run += pr;
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx[j][b], pr, o[b], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
@@ -684,7 +726,7 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
     // computed again in f32.
     float down = kPartDown;   // what a result is to be multiplied with
     if (__builtin_amdgcn_ballot_w64(q_code > kQueryCodes || !finite(o)) != 0) {
-        unit_f32<D, NB, CAUSAL>(p, head, unit, t0, min(t1, wave_tiles), 0, o, m_run, l_run);
+        unit_f32<D, NB, CAUSAL, VEC>(p, head, unit, t0, min(t1, wave_tiles), 0, o, m_run, l_run);
         down = 1.f;
     }
 
@@ -1098,7 +1140,7 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
 
     float down = kPartDown;
     if (__builtin_amdgcn_ballot_w64(!finite(o)) != 0) {
-        unit_f32<D, NB, CAUSAL>(p, head, unit, 0, wave_tiles, dq * DW, o, m_run, l_run);
+        unit_f32<D, NB, CAUSAL, true>(p, head, unit, 0, wave_tiles, dq * DW, o, m_run, l_run);
         down = 1.f;
     }
 

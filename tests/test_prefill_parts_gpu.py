@@ -130,6 +130,26 @@ def test_nan_and_infinity_reach_the_rows_that_see_them(b, d):
     check64(o[:, others], ref[:, others])
 
 
+@pytest.mark.parametrize("b", [1, 4])
+@pytest.mark.parametrize("d", [20, 32, 61, 128])
+def test_recomputed_units_through_strided_dims(b, d):
+    """Views whose dims are a row apart, where the f32 recompute loads one float at
+    a time: keys of minus infinity, and a V at the top of f32's range."""
+    q, k, v = draw(d, b, 40, 20, 97, 300, d)
+    q = np.abs(q) + np.float32(0.01)
+    k[:, 3, 250] = -np.inf
+    v[:, 7] *= np.float32(1e37)
+    nne = T.load_package()
+    dev = [torch.from_numpy(np.ascontiguousarray(x.swapaxes(2, 3))).cuda().transpose(2, 3) for x in (q, k, v)]
+    o = nne.attention_forward(*dev, True, q_offset=203)
+    torch.cuda.synchronize()
+    o = o.cpu().numpy().astype(np.float64)
+    ref = attend64(q, np.maximum(k, np.float32(-1e30)), v, True, 203)
+    for x in (o, ref):
+        x[:, 14:16] *= 1e-37
+    check64(o, ref)
+
+
 def test_row_strides_beyond_the_vector_loads():
     """K/V rows 2^24 floats apart take the scalar-load variant."""
     tk, d, st = 40, 64, 1 << 24
