@@ -1324,28 +1324,45 @@ PrefillSplit prefill_split_plan(PrefillParams& p, bool causal, bool vec) {
         max_t = std::max(max_t, tiles[w]);
     }
     if (max_t < 4) return r;
-    // One or two workgroups per CU (k), and for each the smallest chunk (at most
-    // 16 chunks per item) whose chunks fit.  Two share the CU's matrix cores but
-    // fill each other's waits; more parts cost the last chunk more records.
-    // Fitted to measured calls (us, k = 1 / k = 2, chunk tiles and parts in
-    // brackets): d = 128, 333 rows over 3001 keys 153 [47, 2] / 108 [19, 5], T =
-    // 2610 72 [17, 5] / 66 [8, 11], T = 509 GQA 36 [6, 3] / 39 [3, 6], T = 512
-    // non-causal 30 [4, 4] / 39 [2, 8]; d = 64, T = 3517 61 [28, 4] / 52 [13, 9],
-    // T = 448 19 [4, 4] / 20 [2, 7].  Three per CU were slower than two throughout.
-    const double tile_us[2] = {D == 128 ? 3.1 : 1.7, D == 128 ? 4.6 : 2.4};
-    const double start_us[2] = {D == 128 ? 14.0 : 9.0, D == 128 ? 18.0 : 10.0};
-    const double part_us = D == 128 ? 1.3 : 1.0;
-    int ch = 0;
+    // The chunk of the least cost by a model fitted to 1300 measured calls (11 to 160
+    // key tiles, 1 to 16 heads; within 3 % rms at one workgroup per CU, 7 % at two):
+    // a start, the tiles of a chunk one after the other, and a record per part for
+    // the last chunk to fold.  Two workgroups on a CU share its matrix cores but
+    // fill each other's waits; three were slower throughout.  Measured (us, by
+    // chunk tiles): d = 128, one head, T = 512 26.9 [1], 23.3 [2], 26.0 [4]; 8 heads,
+    // T = 300 21.4 [1], 20.3 [2], 22.7 [3]; 32 heads over 8, T = 509 35.6 [3], 32.9
+    // [6], 35.4 [7]; 16 over 4, B = 2, 333 rows over 3001 keys 118 [10], 103 [18], 139
+    // [40]; d = 32, the same 42.8 [7], 37.4 [12], 59.4 [43].
+    // Candidates: the shortest chunk of each number of parts (at most 16 per item),
+    // and the shortest that leaves one or two workgroups per CU.
+    struct Cost { double tile, start, part; };   // us
+    static constexpr Cost kCost[3][2] = {{{1.2, 6.2, 0.32}, {1.4, 7.2, 0.46}},
+                                         {{1.8, 7.8, 0.52}, {2.1, 10.1, 0.73}},
+                                         {{3.0, 9.7, 0.94}, {3.7, 14.2, 1.33}}};
+    const Cost* cost = kCost[D == 32 ? 0 : D == 64 ? 1 : 2];
+    const auto workgroups = [&](int c) {
+        int64_t n = 0;
+        for (int t : tiles) n += std::max(1, (t + c - 1) / c);
+        return n * p.B * p.Hkv;
+    };
+    int ch = max_t;
     double best = 1e300;
-    for (int k = 1; k <= (D > 32 ? 2 : 1); ++k) {
-        int c = std::max(1, (max_t + 15) / 16);
-        for (;; ++c) {
-            int64_t n = 0;
-            for (int w = 0; w < p.n_wg; ++w) n += std::max(1, (tiles[w] + c - 1) / c);
-            if (n * p.B * p.Hkv <= (int64_t)k * cus || c >= max_t) break;
-        }
-        const double us = tile_us[k - 1] * c + start_us[k - 1] + part_us * ((max_t + c - 1) / c);
+    const auto consider = [&](int c) {
+        const int64_t n = workgroups(c);
+        if (n > 2 * (int64_t)cus) return;
+        const Cost& k = cost[n > cus];
+        const double us = k.tile * c + k.start + k.part * ((max_t + c - 1) / c);
         if (us < best) { best = us; ch = c; }
+    };
+    for (int m = 1; m <= 16; ++m) consider((max_t + m - 1) / m);
+    for (int k = 1; k <= 2; ++k) {
+        int lo = (max_t + 15) / 16, hi = max_t;
+        while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (workgroups(mid) <= (int64_t)k * cus) hi = mid;
+            else lo = mid + 1;
+        }
+        consider(lo);
     }
     const int nc = (max_t + ch - 1) / ch;
     if (nc < 2) return r;

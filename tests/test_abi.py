@@ -312,6 +312,31 @@ def test_workspace_size_queries(nne):
     assert lib.nne_qkv_workspace_size(100, 4, 2, 64, ctypes.byref(size)) == nne.NNE_EINVAL
 
 
+@pytest.mark.parametrize("b,hq,hkv,tq,tk,d,chunk", [
+    # Short prompts on few heads: chunks of two tiles, not one (a record per part
+    # costs the folding chunk more than the second tile).
+    (1, 1, 1, 512, 512, 128, 2), (1, 4, 4, 400, 400, 80, 2), (1, 8, 2, 300, 300, 96, 2),
+    (1, 2, 2, 500, 500, 64, 2), (1, 1, 1, 512, 512, 32, 2),
+    # Chunks that leave one or two workgroups per CU.
+    (1, 32, 8, 509, 509, 128, 6), (2, 16, 4, 333, 3001, 128, 18), (2, 16, 4, 333, 3001, 32, 18),
+])
+def test_prefill_key_split_plan(nne, b, hq, hkv, tq, tk, d, chunk):
+    """The records a causal prefill's key split asks for: (max, sum) of 4 waves x
+    64 lanes and 4 x D/2 x 64 values of O per workgroup, one workgroup per chunk
+    of `chunk` key tiles of each item of 4 units (256 CUs, the count assumed
+    without a device)."""
+    units = hq // hkv * -(-tq // 32)
+    parts = 0
+    for last in range(3, units + 3, 4):
+        row = min(min(last, units - 1) // (hq // hkv) * 32 + 31, tq - 1)
+        parts += -(-(min(row + tk - tq, tk - 1) // 32 + 1) // chunk)
+    size = nne.NneWorkspaceSize()
+    assert nne.lib().nne_attention_workspace_size(i64(b, hq, tq, d), i64(b, hkv, tk, d), 1, tk - tq,
+                                                  ctypes.byref(size)) == nne.NNE_OK
+    padded = next(x for x in (32, 64, 128) if x >= d)
+    assert size.records_bytes == -(-b * hkv * parts // 8) * 8 * (512 + 128 * padded) * 4
+
+
 def test_undersized_caller_workspace_is_refused_before_launch(nne):
     lib = nne.lib()
     lens = np.array([3, 5], np.int32)
