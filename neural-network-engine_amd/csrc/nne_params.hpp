@@ -60,6 +60,9 @@ struct PrefillParams {
     // lengths.  order_cu = 0: items in head-major rank order.
     int order_cu;
     int order_hpx;
+    // Longest first over all heads (order_all): the i-th item of that order is
+    // slot i / 8 of XCD i % 8.
+    int order_all;
     // Key split for problems too small to fill the chip (n_chunks > 1): the
     // key tiles of every work item are cut into chunks of chunk_tiles tiles,
     // one workgroup per (item, chunk); each leaves a partial (max, sum, O)

@@ -77,6 +77,13 @@ __device__ __forceinline__ int last_visible_key(const PrefillParams& p, int rb, 
 // missing partner of an odd middle rank, 1 with (head, wgi) otherwise.
 __device__ __forceinline__ int item_at(const PrefillParams& p, int j, int x, int q, int S, int& head,
                                        int& wgi) {
+    if (p.order_all) {
+        const int heads = p.B * p.Hkv, i = 8 * q + x;
+        if (j > 0 || i >= heads * p.n_wg) return 0;
+        head = i % heads;
+        wgi = p.n_wg - 1 - i / heads;
+        return 1;
+    }
     if (p.order_cu) {
         // Position pos in the XCD's items sorted longest first (rank-major over
         // its heads).  The hardware places workgroup q of an XCD on CU q % h
@@ -1232,6 +1239,22 @@ int persistent_slots(PrefillParams& p, bool causal, int cus, int k_max) {
     // 1016 to 592 us and B = 1, Hq = 32, Hkv = 8, T = 2048 from 401 to 296 us.
     p.order_cu = 0;
     p.order_hpx = 0;
+    p.order_all = 0;
+    // One workgroup per CU and more items than CUs: the order above would give the
+    // CUs that finish first the shortest items left and leave the longest running
+    // alone, and pairs that do not fill their last round idle up to half the CUs.
+    // All heads' items, longest first, as CUs get free (us; the deep kernel): d =
+    // 320, 14 heads, T = 2300 743 -> 442 (679), 17 heads, T = 1024 231 -> 183 (220), 2 KV
+    // heads of 16, T = 700 216 -> 128 (205); d = 192, 48 heads, T = 1500 440 -> 284, 9
+    // heads, T = 6000 1258 -> 800.  Pairs that fill their rounds keep a head's K/V in
+    // one XCD's L2: d = 512, 16 heads, T = 2048 493 against 505.
+    const int64_t items = heads * p.n_wg;
+    if (causal && k_max == 1 && items > cus && items < INT32_MAX - 8 &&
+        (!p.pairing || (double)p.per_xcd / ((double)((p.per_xcd + cu_per_xcd - 1) / cu_per_xcd) * cu_per_xcd) < 0.9)) {
+        p.pairing = 0;
+        p.order_all = 1;
+        return (int)((items + 7) / 8);
+    }
     if (causal && !p.pairing && S == p.per_xcd && heads % 8 == 0 && cu_per_xcd > 0 &&
         (int64_t)p.per_xcd * 8 == heads * p.n_wg) {
         p.order_cu = cu_per_xcd;

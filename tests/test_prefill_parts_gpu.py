@@ -64,6 +64,15 @@ def test_tile_edges_above_128_dims(d, hq, hkv, tq, tk, causal):
     check64(run(q, k, v, causal, tk - tq), attend64(q, k, v, causal, tk - tq))
 
 
+# More workgroups than CUs, causal: items longest first over all heads (the heads no
+# multiple of 8, the items none either), and pairs with a last round barely filled.
+@pytest.mark.parametrize("d,hq,hkv,t", [(132, 301, 301, 140), (256, 270, 135, 130), (260, 300, 300, 65),
+                                        (388, 61, 61, 290), (512, 66, 11, 225), (320, 42, 42, 449)])
+def test_causal_items_longest_first(d, hq, hkv, t):
+    q, k, v = draw(d + t, 1, hq, hkv, t, t, d)
+    check64(run(q, k, v, True), attend64(q, k, v, True))
+
+
 @pytest.mark.parametrize("d", [256, 512])
 @pytest.mark.parametrize("qs,ks,vs", [(1.0, 1.0, 1e-37), (1e-30, 1e30, 1.0), (1e30, 1e-30, 1.0)])
 def test_magnitudes_above_128_dims(d, qs, ks, vs):
