@@ -223,21 +223,14 @@ int deep_workspace(nne::DeepParams& p, int max_tiles, const nne_workspace_t* wsp
     return NNE_OK;
 }
 
-// Head dims 129-512 with more query rows per KV head than the split-K kernel
-// takes: the 8-wave kernel when there are more 32-row units than CUs (above
-// 256 dims, causal: than two per CU, whose lengths then even out), else the
-// deep kernel, which spreads or key-splits them over every CU.  Measured on
-// both sides (deep / 8-wave, us): d = 256, T = 1024, 8 heads (256 units) 164 /
-// 163 and 10 heads 273 / 173; T = 64, 128 heads (256 units) 18 / 20; d = 512
-// non-causal, T = 512, 16 heads (256 units) 88 / 120, T = 1024, 10 heads (320)
-// 292 / 227; causal, T = 1024, 16 heads (512 units) 178 / 228, 20 heads (640)
-// 323 / 296, T = 4096, 16 heads 2414 / 2007.
-bool on_deep(int64_t B, int64_t Hkv, int64_t G, int64_t Tq, int d, bool causal) {
+// Whether a problem runs on the deep kernel: above 512 dims, and at 129-512 with
+// more query rows per KV head than the split-K kernel takes (up to 256 dims),
+// where deep_prefill_faster puts it.
+bool on_deep(int64_t B, int64_t Hkv, int64_t G, int64_t Tq, int64_t Tk, int d, bool causal, int64_t qoff) {
     if (nne::prefill_padded_dim(d) != 0) return false;
     if (d > 512) return true;
     if (G * Tq <= nne::splitk_max_rows()) return nne::splitk_padded_dim(d) == 0;
-    const int64_t units = B * Hkv * G * ((Tq + 31) / 32);
-    return units <= (int64_t)device_cus() * (d > 256 && causal ? 2 : 1);
+    return nne::deep_prefill_faster(B * Hkv, G, Tq, Tk, d, causal, qoff, device_cus());
 }
 
 // Records of the largest key split a deep-kernel problem of these shapes
@@ -276,10 +269,10 @@ int run_attention(const float* q, const int64_t* qs_, const int64_t* qst, const 
     const bool deep_strides = kst[2] >= 0 && vst[2] >= 0 && kst[2] < (1 << 25) && vst[2] < (1 << 25);
     const bool wide_strides = kst[2] >= 0 && vst[2] >= 0 && kst[2] < nne::kMaxTileStride &&
                               vst[2] < nne::kMaxTileStride;
-    const bool deep = wide && (d > 256 ? !wide_strides || on_deep(B, Hkv, Hq / Hkv, Tq, d, causal)
-                                       : deep_strides && on_deep(B, Hkv, Hq / Hkv, Tq, d, causal));
     // Offsets beyond +-2^30 cannot change visibility for int32 lengths.
     const int qoff = (int)std::max<int64_t>(-(1 << 30), std::min<int64_t>(q_offset, 1 << 30));
+    const bool deep_rule = wide && on_deep(B, Hkv, Hq / Hkv, Tq, Tk, d, causal, qoff);
+    const bool deep = wide && (d > 256 ? !wide_strides || deep_rule : deep_strides && deep_rule);
     const bool vec = d % 4 == 0 && vec_view(q, qst) && vec_view(k, kst) && vec_view(v, vst) &&
                      vec_view(o, ost);
     if (wide && !vec)
@@ -425,7 +418,7 @@ nne_workspace_size_t attention_workspace(const int64_t* qs_, const int64_t* ks_,
     const int qoff = (int)std::max<int64_t>(-(1 << 30), std::min<int64_t>(q_offset, 1 << 30));
     // The deep kernel's key split: above 256 dims, and head dims 129-256 on its
     // 2-wave form.
-    if (nne::splitk_padded_dim(d) == 0 || (Hq % Hkv == 0 && on_deep(B, Hkv, Hq / Hkv, Tq, d, causal))) {
+    if (nne::splitk_padded_dim(d) == 0 || (Hq % Hkv == 0 && on_deep(B, Hkv, Hq / Hkv, Tq, Tk, d, causal, qoff))) {
         if (d % 4 == 0 && Hq % Hkv == 0)
             r.records_bytes = deep_workspace_bytes(B, Hq, Hkv, Tq, d, deep_max_tiles(Tk, causal, qoff, Tq));
         return r;

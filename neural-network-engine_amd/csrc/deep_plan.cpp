@@ -1,5 +1,7 @@
-// Key-split plans of the deep kernel (deep.hip), host side, plain C++.
+// Plans of the deep kernel (deep.hip), host side, plain C++.
 #include "deep_plan.hpp"
+
+#include <algorithm>
 
 namespace nne {
 
@@ -91,6 +93,44 @@ uint64_t deep_ragged_plan(DeepParams& p, const int32_t* seq_keys, int cus, uint6
     p.n_split = kDeepMaxSplit;   // marks a split launch; parts per pair come from part_prefix
     p.split_tiles = (int)target;
     return bytes;
+}
+
+// With at most as many 32-row units as CUs (causal above 256 dims: two per CU,
+// whose lengths even out) the deep kernel spreads or key-splits them over every
+// CU, where the 8-wave kernel would leave most idle (deep / 8-wave, us: d = 256, T =
+// 1024, 8 heads 164 / 163; T = 64, 128 heads 18 / 20; d = 512 non-causal, T = 512, 16
+// heads 88 / 120; causal, T = 1024, 16 heads 178 / 228).  With more, the 8-wave
+// kernel is 1.25 to 1.8 times as fast per unit and tile while its workgroups of 4
+// units of one KV head (2 above 256 dims), one per CU, are full; KV heads of few
+// units leave waves without a unit, and a few workgroups past a round of the CUs
+// cost another round.  So the time of each is estimated as rounds of its
+// workgroups (deep: 4 units at once on a CU, 2 above 256 dims), each a start and
+// its tiles; the constants are fitted to calls of 257 to 3000 units, all measured
+// on both (deep / 8-wave): d = 192, 300 heads of 65 rows 33 / 42, of 65 over 333 keys 89
+// / 102, 600 of 40 rows 42 / 47, 90 of 100 34 / 25; d = 256, 257 heads of 32 rows 16 / 33;
+// d = 320, 300 heads of 65 58 / 77, causal 51 / 67, 9 of 1024 222 / 183; d = 512, 257 of
+// 32 over 1000 keys 355 / 484, 100 of 96 over 1000 319 / 241.  Estimates within 10 %
+// keep the 8-wave kernel (d = 508, 150 heads of 530 rows over 42 keys 219 / 194).
+bool deep_prefill_faster(int64_t heads, int64_t G, int64_t Tq, int64_t Tk, int d, bool causal,
+                         int64_t q_offset, int cus) {
+    const int64_t units = G * ((Tq + 31) / 32);
+    if (heads * units <= (int64_t)cus * (d > 256 && causal ? 2 : 1)) return true;
+    struct Cost { double start, tile; };   // us
+    static constexpr Cost kWide[4] = {{7.5, 4.1}, {12.0, 4.7}, {8.0, 5.6}, {11.5, 7.05}};
+    static constexpr Cost kDeep[4] = {{6.6, 7.1}, {8.5, 8.0}, {6.5, 7.0}, {10.0, 9.0}};
+    const int at = d <= 192 ? 0 : d <= 256 ? 1 : d <= 384 ? 2 : 3;
+    const auto tiles_of = [&](int64_t unit) {
+        const int64_t keys = causal ? std::min(Tk, std::min((unit / G + 1) * 32, Tq) + q_offset) : Tk;
+        return (double)((std::max<int64_t>(keys, 0) + 31) / 32);
+    };
+    // (The deep kernel's units run across the query heads of a KV head.)
+    const auto us = [&](const Cost& c, int64_t per_wg, int64_t slots) {
+        const int64_t n = heads * (per_wg > 1 ? (units + per_wg - 1) / per_wg : (G * Tq + 31) / 32);
+        const double first = tiles_of(std::min(per_wg, units) - 1), last = tiles_of(units - 1);
+        const double rounds = (double)((n + slots - 1) / slots);
+        return rounds * c.start + c.tile * std::max({last, rounds * first, n * (first + last) / 2 / slots});
+    };
+    return us(kDeep[at], 1, (int64_t)cus * (d <= 256 ? 4 : 2)) < 0.9 * us(kWide[at], d <= 256 ? 4 : 2, cus);
 }
 
 }  // namespace nne

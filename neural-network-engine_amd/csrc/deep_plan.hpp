@@ -1,5 +1,5 @@
-// Host-side key-split plans of the deep kernel (head dims above 256, deep.hip):
-// plain C++ (no HIP), shared by the C ABI and the planner's CPU tests.
+// Host-side plans of the deep kernel (deep.hip): key splits, and which prefill it
+// takes.  Plain C++ (no HIP), shared by the C ABI and the planner's CPU tests.
 #pragma once
 
 #include <stdint.h>
@@ -18,5 +18,9 @@ uint64_t deep_split_plan(DeepParams& p, int max_tiles, int cus, uint64_t max_byt
 // returns the record bytes, or 0 (p.ragged = 0) when the step does not gain
 // from it.
 uint64_t deep_ragged_plan(DeepParams& p, const int32_t* seq_keys, int cus, uint64_t max_bytes);
+// Whether a prefill at 129-512 dims (heads: B * Hkv) takes the deep kernel and
+// not the 8-wave kernel of prefill.hip.
+bool deep_prefill_faster(int64_t heads, int64_t G, int64_t Tq, int64_t Tk, int d, bool causal,
+                         int64_t q_offset, int cus);
 
 }  // namespace nne

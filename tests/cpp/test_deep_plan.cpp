@@ -12,6 +12,9 @@
 //   * equal split: none unless at most half as many workgroups as CUs and
 //     8+ tiles; at most kDeepMaxSplit parts of at least 4 tiles covering the
 //     longest unit, all parts in one round, records within max_bytes.
+//   * deep_prefill_faster: calls measured on both kernels go to the faster one
+//     (at least 5 % apart), and rounds of the device scale (twice the CUs and
+//     heads change nothing).
 // Prints "<failed> of <checks> checks failed" and exits non-zero on failure.
 #include <algorithm>
 #include <cstdio>
@@ -150,7 +153,51 @@ static void check_split(int B, int Hkv, int G, int Tq, int d, int max_tiles, int
               (long long)cap);
 }
 
+struct Route { int heads, G, Tq, Tk, d; bool causal, deep; };
+
+static void check_routes() {
+    const Route routes[] = {
+        // KV heads of few units, or a few workgroups past a round
+        {257, 1, 32, 32, 192, false, true},   {300, 1, 33, 33, 132, true, true},
+        {300, 1, 65, 65, 192, false, true},   {300, 1, 65, 333, 200, false, true},
+        {257, 1, 32, 1000, 192, false, true}, {600, 1, 40, 40, 192, false, true},
+        {300, 1, 33, 33, 256, false, true},   {257, 1, 32, 32, 260, false, true},
+        {300, 1, 65, 65, 384, false, true},   {300, 1, 65, 65, 320, true, true},
+        {300, 1, 65, 65, 512, true, true},    {257, 1, 32, 1000, 512, false, true},
+        {300, 1, 65, 333, 448, false, true},
+        // at most one unit per CU (causal above 256 dims: two)
+        {8, 1, 1024, 1024, 256, true, true},  {16, 1, 1024, 1024, 512, true, true},
+        // the rest
+        {130, 1, 64, 64, 192, false, false},  {90, 1, 100, 100, 132, true, false},
+        {9, 1, 1024, 1024, 192, true, false}, {100, 1, 96, 2000, 192, false, false},
+        {2, 16, 300, 300, 256, true, false},  {16, 4, 160, 160, 200, false, false},
+        {160, 1, 1500, 1500, 192, false, false}, {16, 1, 4096, 4096, 256, true, false},
+        {9, 1, 1024, 1024, 320, false, false}, {100, 1, 96, 1000, 448, false, false},
+        {14, 1, 2300, 2300, 320, true, false}, {17, 1, 1024, 1024, 512, true, false},
+        {40, 1, 512, 512, 260, true, false},  {16, 1, 4096, 4096, 512, true, false},
+        {16, 1, 2048, 2048, 384, false, false}, {8, 8, 300, 300, 512, true, false},
+        {150, 1, 530, 42, 508, false, false},
+    };
+    for (const Route& r : routes) {
+        char buf[160];
+        std::snprintf(buf, sizeof buf, "route heads=%d G=%d Tq=%d Tk=%d d=%d causal=%d", r.heads, r.G, r.Tq,
+                      r.Tk, r.d, r.causal);
+        g_case = buf;
+        const int64_t off = r.causal ? r.Tk - r.Tq : 0;
+        CHECK(deep_prefill_faster(r.heads, r.G, r.Tq, r.Tk, r.d, r.causal, off, 256) == r.deep,
+              "expected deep = %d", r.deep);
+        CHECK(deep_prefill_faster(2 * r.heads, r.G, r.Tq, r.Tk, r.d, r.causal, off, 512) == r.deep,
+              "twice the heads and CUs: expected deep = %d", r.deep);
+    }
+    // No key visible to any row, and no keys at all: either kernel, no overflow.
+    g_case = "route without keys";
+    CHECK(deep_prefill_faster(1, 1, 8, 8, 192, true, -(1 << 30), 256), "few units");
+    deep_prefill_faster(INT32_MAX / 64, 1, 64, 0, 512, true, -(1 << 30), 256);
+    deep_prefill_faster(1, 1, INT32_MAX, INT32_MAX, 132, true, 1 << 30, 256);
+}
+
 int main() {
+    check_routes();
     // Named cases: the benchmark-like decode batches, and more pairs than CUs
     // (B = 64, Hkv = 8 on 256 CUs: 512 pairs), which must return at once.
     std::mt19937 rng(7);
