@@ -263,16 +263,14 @@ int run_attention(const float* q, const int64_t* qs_, const int64_t* qst, const 
     // (on_deep), or up to 256 dims on the split-K kernel when a KV head has few
     // query rows.
     const bool wide = nne::prefill_padded_dim(d) == 0;
-    // K/V row strides outside the deep kernel's 32-bit tile offsets keep the
-    // 8-wave kernel up to 256 dims; strides outside that kernel's vector loads
-    // keep the deep kernel above.
-    const bool deep_strides = kst[2] >= 0 && vst[2] >= 0 && kst[2] < (1 << 25) && vst[2] < (1 << 25);
-    const bool wide_strides = kst[2] >= 0 && vst[2] >= 0 && kst[2] < nne::kMaxTileStride &&
+    // K/V row strides outside the 32-bit tile offsets of the deep kernel and of the
+    // 8-wave kernel's vector loads take that kernel's scalar loads up to 256 dims
+    // and are refused above.
+    const bool tile_strides = kst[2] >= 0 && vst[2] >= 0 && kst[2] < nne::kMaxTileStride &&
                               vst[2] < nne::kMaxTileStride;
     // Offsets beyond +-2^30 cannot change visibility for int32 lengths.
     const int qoff = (int)std::max<int64_t>(-(1 << 30), std::min<int64_t>(q_offset, 1 << 30));
-    const bool deep_rule = wide && on_deep(B, Hkv, Hq / Hkv, Tq, Tk, d, causal, qoff);
-    const bool deep = wide && (d > 256 ? !wide_strides || deep_rule : deep_strides && deep_rule);
+    const bool deep = wide && (tile_strides ? on_deep(B, Hkv, Hq / Hkv, Tq, Tk, d, causal, qoff) : d > 256);
     const bool vec = d % 4 == 0 && vec_view(q, qst) && vec_view(k, kst) && vec_view(v, vst) &&
                      vec_view(o, ost);
     if (wide && !vec)
@@ -280,8 +278,7 @@ int run_attention(const float* q, const int64_t* qs_, const int64_t* qst, const 
                                 "multiple of 4, unit dim strides, strides that are multiples of 4 "
                                 "and 16-byte aligned tensors", d);
     if (deep) {
-        // The deep kernel addresses 32 K/V rows of a tile with 32-bit byte offsets.
-        if (kst[2] < 0 || vst[2] < 0 || kst[2] >= (1 << 25) || vst[2] >= (1 << 25))
+        if (!tile_strides)
             return fail(NNE_EINVAL, "Invalid configuration or argument: K/V row strides must lie in "
                                     "[0, 2^25) floats at head dim %d", d);
         nne::DeepParams p{};

@@ -33,7 +33,9 @@ struct OutView4 {
 // 4w .. 4w+3, so the G query heads of a group share every K/V tile the
 // workgroup stages in LDS.
 constexpr int kMaxSplitItems = 256;   // work items per KV head of a key-split launch
-constexpr int64_t kMaxTileStride = 1 << 24;   // K/V row strides (floats) below this, from 0, are read as vectors
+// K/V row strides (floats) below this, from 0, are read as vectors: 31 rows and a
+// row's dims stay within a 32-bit byte offset.
+constexpr int64_t kMaxTileStride = 1 << 25;
 
 struct PrefillParams {
     View4 q, k, v;

@@ -145,7 +145,7 @@ struct SplitTile {
     static_assert(KR % RPI == 0 && LPR <= 64 * NC, "whole rows per load");
     float4 kr[NK];
     float vr[NJ][8];
-    // VEC views (row strides in [0, 2^24)): byte offsets of this lane within a
+    // VEC views (row strides in [0, kMaxTileStride)): byte offsets of this lane within a
     // tile and of each load's rows, so that a tile's loads need only its base.
     uint32_t k_lane[NC], k_step, v_lane[NJ], v_row0, v_st;
 

@@ -159,10 +159,15 @@ def test_recomputed_units_through_strided_dims(b, d):
     check64(o, ref)
 
 
-def test_row_strides_beyond_the_vector_loads():
-    """K/V rows 2^24 floats apart take the scalar-load variant."""
-    tk, d, st = 40, 64, 1 << 24
-    q, k, v = draw(10, 1, 2, 1, 64, tk, d)
+# The last stride of the vector loads' 32-bit offsets, and the first of the scalar
+# loads; few units (up to 128 dims the key split), and more than CUs.
+@pytest.mark.parametrize("d,heads,st", [(64, 2, 1 << 24), (64, 2, (1 << 25) - 4), (64, 2, 1 << 25),
+                                        (192, 300, (1 << 25) - 4), (192, 300, 1 << 25),
+                                        (512, 300, (1 << 25) - 4)])
+def test_row_strides_beyond_the_vector_loads(d, heads, st):
+    """K/V rows 2^25 floats apart take the scalar-load variant."""
+    tk = 40
+    q, k, v = draw(10, 1, heads, 1, 64, tk, d)
     big = torch.empty(tk * st, device="cuda")
     kd, vd = (torch.as_strided(big, (1, 1, tk, d), (tk * st, tk * st, st, 1), off) for off in (0, 512))
     kd.copy_(torch.from_numpy(k))
