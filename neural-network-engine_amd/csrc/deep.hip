@@ -191,16 +191,18 @@ __global__ __launch_bounds__(64 * DW, DW == 8 ? 1 : 2) void deep_attention_kerne
     const int od = oc * CB * OB + 32 * wave + l32;   // this lane's dim of output block 0
 
     // K and V of a tile are read through buffer ranges that start at the
-    // tile's first key and end with the last key of the unit (rows past it
-    // read as zero without a memory access), so no load needs a predicate
-    // and the byte offsets are a lane constant plus a small uniform part.
-    // K columns past d (the odd half of a last 8-dim chunk when d % 8 == 4)
-    // are read from memory next to the row and zeroed; V columns past d read
+    // tile's first key and end with the dims of the unit's last key (rows past
+    // it read as zero without a memory access, or where rows overlap as part of
+    // other rows, at no weight), so no load needs a predicate and the byte
+    // offsets are a lane constant plus a small uniform part.  K columns past d
+    // (the odd half of a last 8-dim chunk when d % 8 == 4) are read from memory
+    // next to the row and zeroed; V columns past d read
     // the row's last float and only reach O columns never stored.
     auto range = [&](const float* base, int64_t st, int key0) {
         const int nk = kend - key0 < 32 ? kend - key0 : 32;
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + key0 * st), 0,
-                                                 (uint32_t)nk * (uint32_t)st * 4u, 0x00020000);
+                                                 nk > 0 ? ((uint32_t)(nk - 1) * (uint32_t)st + (uint32_t)p.d) * 4u : 0u,
+                                                 0x00020000);
     };
     const uint32_t k_lane = ((uint32_t)l32 * (uint32_t)p.k.st + 8 * wave + 4 * half) * 4u;
     auto load_k = [&](__amdgpu_buffer_rsrc_t rk, int i) -> vf4 {

@@ -489,10 +489,13 @@ __global__ __launch_bounds__(256, (D >= 128 && ROWS >= 16) ? 1 : 2) void splitk_
         // the caches' normal allocation lifts a chunked read of the cache from
         // ~6.0 to ~6.9 TB/s on MI355X.  (The host keeps a head under 2^30
         // floats, so the byte offsets fit in 32 bits.)
-        const __amdgpu_buffer_rsrc_t krange = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(kb), 0, (uint32_t)key_end * (uint32_t)kst * 4u, 0x00020000);
-        const __amdgpu_buffer_rsrc_t vrange = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(vb), 0, (uint32_t)key_end * (uint32_t)vst * 4u, 0x00020000);
+        // A range ends with its last row's dims, also where rows overlap or are all
+        // the same (row strides below d).
+        const auto range = [&](const float* base, int st) {
+            const uint32_t bytes = key_end > 0 ? ((uint32_t)(key_end - 1) * (uint32_t)st + (uint32_t)p.d) * 4u : 0u;
+            return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00020000);
+        };
+        const __amdgpu_buffer_rsrc_t krange = range(kb, kst), vrange = range(vb, vst);
         // Byte offset = a lane constant + a wave-uniform part per load (one
         // VALU add each; no per-load address registers live across blocks).
         const uint32_t k_lane = ((uint32_t)(lane / LPR) * (uint32_t)kst + (uint32_t)kc_col) * 4u;

@@ -241,3 +241,20 @@ def test_results_far_below_one_on_ordinary_values(d):
     ref = attend64(q, k, v, False)
     seen = ref > 2.0**-124
     assert (np.abs(run(q, k, v, False) - ref)[seen] <= 16 * 2.0**-18 * np.log(2) * ref[seen]).all()
+
+
+@pytest.mark.parametrize("d,heads,tq", [(64, 2, 4), (128, 8, 16), (192, 2, 3), (256, 4, 16),      # split-K
+                                        (64, 4, 40), (128, 20, 300), (192, 4, 70), (512, 4, 40)])
+@pytest.mark.parametrize("step", [0, 4])
+def test_rows_that_overlap(d, heads, tq, step):
+    """K/V views whose rows are one row broadcast (row stride 0) or a window that
+    moves by 4 floats."""
+    tk = 90
+    rng = np.random.default_rng(d + step)
+    kf, vf = (rng.standard_normal(step * tk + d).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((1, heads, tq, d)).astype(np.float32)
+    rows = np.arange(tk)[:, None] * step + np.arange(d)
+    kd, vd = (torch.as_strided(torch.from_numpy(x).cuda(), (1, 1, tk, d), (0, 0, step, 1)) for x in (kf, vf))
+    o = T.load_package().attention_forward(torch.from_numpy(q).cuda(), kd, vd, False)
+    torch.cuda.synchronize()
+    check64(o.cpu().numpy(), attend64(q, kf[rows][None, None], vf[rows][None, None], False))
