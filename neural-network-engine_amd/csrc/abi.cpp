@@ -305,10 +305,12 @@ int run_attention(const float* q, const int64_t* qs_, const int64_t* qst, const 
     // qoff < tk - 1.
     const int64_t tk = causal ? std::max<int64_t>(0, std::min<int64_t>(Tk, (int64_t)qoff + Tq)) : Tk;
     const bool masked = causal && (int64_t)qoff < tk - 1;
-    // The split-K kernel addresses a head's rows with 32-bit byte offsets.
-    const bool fits32 = (int64_t)B * Hkv * Tk < INT32_MAX && (int64_t)Tk * kst[2] < (1LL << 30) &&
+    // The split-K kernel addresses a head's rows with 32-bit byte offsets from
+    // its first one: rows that run backwards go to the other kernels.
+    const bool forward = kst[2] >= 0 && vst[2] >= 0;
+    const bool fits32 = forward && (int64_t)B * Hkv * Tk < INT32_MAX && (int64_t)Tk * kst[2] < (1LL << 30) &&
                         (int64_t)Tk * vst[2] < (1LL << 30);
-    if (wide && rows > nne::splitk_max_rows()) {
+    if (wide && (rows > nne::splitk_max_rows() || !forward)) {
         nne::PrefillParams p{};
         p.q = make_view(q, qst);
         p.k = make_view(k, kst);

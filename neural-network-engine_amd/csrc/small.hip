@@ -318,7 +318,8 @@ hipError_t launch_small_d(const PrefillParams& p, bool causal, int cus, hipStrea
 bool small_prefill_fits(const PrefillParams& p, bool vec, int cus) {
     if (!vec || p.d % 4 != 0 || p.d > 128 || p.Hkv == 0) return false;
     // key offsets are 32-bit in the kernel
-    if ((int64_t)p.Tk * p.k.st >= INT32_MAX || (int64_t)p.Tk * p.v.st >= INT32_MAX) return false;
+    if ((int64_t)p.Tk * std::max(p.k.st, -p.k.st) >= INT32_MAX || (int64_t)p.Tk * std::max(p.v.st, -p.v.st) >= INT32_MAX)
+        return false;
     const int64_t wgs = (int64_t)p.B * p.Hq * ((p.Tq + SKB - 1) / SKB);
     // Tiles of the heaviest row block: at most two per wave.
     const int64_t tiles = ((int64_t)p.Tk + SKB - 1) / SKB;

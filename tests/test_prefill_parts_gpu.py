@@ -258,3 +258,28 @@ def test_rows_that_overlap(d, heads, tq, step):
     o = T.load_package().attention_forward(torch.from_numpy(q).cuda(), kd, vd, False)
     torch.cuda.synchronize()
     check64(o.cpu().numpy(), attend64(q, kf[rows][None, None], vf[rows][None, None], False))
+
+
+# Few rows (split-K, were the rows in order), few units, and more units than CUs;
+# the scalar loads of every kernel that takes such rows, over several key tiles.
+@pytest.mark.parametrize("d,heads,tq,tk", [(64, 2, 4, 90), (128, 8, 16, 300), (64, 4, 40, 200), (128, 20, 97, 289),
+                                           (192, 2, 3, 90), (256, 4, 16, 100), (132, 3, 70, 100),
+                                           (192, 300, 40, 109), (256, 130, 97, 129)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_rows_that_run_backwards(d, heads, tq, tk, causal):
+    """Negative K/V row strides through the C ABI (torch has none)."""
+    import ctypes
+    nne = T.load_package()
+    q, k, v = draw(d + tk, 1, heads, heads, tq, tk, d)
+    dev = [torch.from_numpy(x).cuda() for x in (q, k[:, :, ::-1].copy(), v[:, :, ::-1].copy())]
+    o = torch.full(q.shape, float("nan"), device="cuda")
+    i64 = ctypes.c_int64 * 4
+    rows = i64(heads * tk * d, tk * d, -d, 1)
+    last = (tk - 1) * d * 4          # row 0 of the reversed tensors
+    args = []
+    for t, first, st in ((dev[0], 0, None), (dev[1], last, rows), (dev[2], last, rows)):
+        args += [ctypes.c_void_p(t.data_ptr() + first), i64(*t.shape), st]
+    nne.check(nne.lib().nne_attention_forward(*args, ctypes.c_void_p(o.data_ptr()), None, int(causal), tk - tq,
+                                              0, 0.0, None))
+    torch.cuda.synchronize()
+    check64(o.cpu().numpy(), attend64(q, k, v, causal, tk - tq))
