@@ -26,6 +26,8 @@ bool plan_packing(SplitKParams& p, int slots, int64_t total_keys);
 // or max_wg + 1 if it needs more workgroups or gives a head more than
 // max_parts of them.
 int cut_chunks(const SplitKParams& p, int64_t x, int64_t ovh, int max_wg, int* ends);
+// The least keys of a chunk (cut and equal chunks), longest head max_len.
+int64_t shortest_chunk(int d, int max_len);
 // Cut chunks (fused launches with the prefix in the arguments): sets cut,
 // chunk, n_wg, chunk_end.
 bool plan_cut(SplitKParams& p, int slots, int64_t total_keys, int max_len);

@@ -146,6 +146,7 @@ static char check_layout(const Shape& s) {
     } else {
         mode = 'e';
         CHECK(p.chunk % kKeyBlock == 0 && p.chunk >= kKeyBlock, "chunk %d", p.chunk);
+        CHECK(p.chunk >= shortest_chunk(s.d, (int)max_len), "chunk %d below the shortest", p.chunk);
         CHECK((int64_t)p.n_wg * p.chunk >= total && (int64_t)(p.n_wg - 1) * p.chunk < total,
               "n_wg %d x chunk %d vs %lld keys", p.n_wg, p.chunk, (long long)total);
         for (int w = 0; w < p.n_wg; ++w) start.push_back((int64_t)w * p.chunk);
@@ -200,10 +201,11 @@ static char check_layout(const Shape& s) {
         }
         for (size_t h = 0; h < heads.size(); ++h)
             CHECK(parts[h] <= p.max_parts, "head %zu in %d workgroups > %d", h, parts[h], p.max_parts);
-        // The smallest budget: one key less needs more workgroups (or breaks
-        // the floor of 4 blocks / an eighth of the longest head).
-        const int64_t floor_x = std::max<int64_t>((total + s.slots - 1) / s.slots,
-                                                  std::max<int64_t>(4 * kKeyBlock, (max_len + 7) / 8));
+        // The smallest budget: one key less needs more workgroups, or breaks
+        // the floor of the shortest chunk.
+        const int64_t shortest = shortest_chunk(s.d, (int)max_len);
+        const int64_t floor_x = std::max<int64_t>((total + s.slots - 1) / s.slots, shortest);
+        CHECK(x >= shortest, "budget %lld below the shortest chunk %lld", (long long)x, (long long)shortest);
         if (x > floor_x)
             CHECK(cut_chunks(p, x - 1, ovh, std::min(s.slots, kMaxCutWg), nullptr) > std::min(s.slots, kMaxCutWg),
                   "budget %lld not minimal", (long long)x);
@@ -211,7 +213,42 @@ static char check_layout(const Shape& s) {
     return mode;
 }
 
+// The shortest chunk on both sides of its lines: a block for each of 4 waves, an
+// eighth of the head, 160 KB of K and V rows, a 32nd of the head (past 5 MB).
+static void check_shortest_chunk() {
+    const int cases[][3] = {   // d, longest head, keys
+        {128, 1, 64},     {128, 512, 64},    {128, 513, 65},    {128, 1272, 159},  {128, 1280, 160},
+        {128, 1733, 160}, {128, 5120, 160},  {128, 5121, 161},  {128, 8000, 250},  {64, 2552, 319},
+        {64, 3000, 320},  {64, 10240, 320},  {64, 10241, 321},  {256, 100, 64},    {256, 632, 79},
+        {256, 1000, 80},  {256, 2561, 81},   {32, 5000, 625},   {32, 6000, 640},   {128, 1 << 20, 32768},
+    };
+    for (const auto& c : cases) {
+        g_case = "shortest chunk d=" + std::to_string(c[0]) + " keys=" + std::to_string(c[1]);
+        const int64_t got = shortest_chunk(c[0], c[1]);
+        CHECK(got == c[2], "%lld, expected %d", (long long)got, c[2]);
+    }
+    // Long heads on few workgroups: the budget is the shortest chunk, and a head
+    // takes the parts it gives.
+    struct Long { int Hkv, R, d, len, budget, parts; } longs[] = {
+        {8, 4, 128, 1733, 160, 11}, {2, 8, 128, 4000, 160, 25}, {8, 4, 128, 8000, 250, 32},
+        {4, 8, 64, 3000, 320, 10},  {2, 4, 256, 2000, 80, 25},
+    };
+    for (const Long& l : longs) {
+        Shape s{1, l.Hkv, l.d, l.R, {l.len}, 256};
+        g_case = "long head d=" + std::to_string(l.d) + " keys=" + std::to_string(l.len);
+        CHECK(check_layout(s) == 'c', "not cut");
+        SplitKParams p;
+        setup(p, s);
+        plan_split_layout(p, s.slots, (int64_t)l.Hkv * l.len, l.len);
+        CHECK(p.chunk == l.budget, "budget %d, expected %d", p.chunk, l.budget);
+        const int per_head = (p.n_wg + l.Hkv - 1) / l.Hkv;
+        CHECK(per_head == l.parts || per_head == l.parts + 1, "%d workgroups for %d heads, expected %d a head", p.n_wg,
+              l.Hkv, l.parts);
+    }
+}
+
 int main() {
+    check_shortest_chunk();
     // Named shapes: the mode the measurements chose for each.
     struct Named {
         const char* name;
