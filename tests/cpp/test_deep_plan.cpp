@@ -153,7 +153,7 @@ static void check_split(int B, int Hkv, int G, int Tq, int d, int max_tiles, int
               (long long)cap);
 }
 
-struct Route { int heads, G, Tq, Tk, d; bool causal, deep; };
+struct Route { int heads, G, Tq, Tk, d; bool causal, deep; int off = INT32_MIN; };
 
 static void check_routes() {
     const Route routes[] = {
@@ -164,7 +164,8 @@ static void check_routes() {
         {300, 1, 33, 33, 256, false, true},   {257, 1, 32, 32, 260, false, true},
         {300, 1, 65, 65, 384, false, true},   {300, 1, 65, 65, 320, true, true},
         {300, 1, 65, 65, 512, true, true},    {257, 1, 32, 1000, 512, false, true},
-        {300, 1, 65, 333, 448, false, true},
+        {300, 1, 65, 333, 448, false, true}, {257, 1, 65, 115, 260, true, true},
+        {300, 1, 65, 65, 388, true, true, -10}, {257, 1, 32, 300, 512, false, true},
         // at most one unit per CU (causal above 256 dims: two)
         {8, 1, 1024, 1024, 256, true, true},  {16, 1, 1024, 1024, 512, true, true},
         // the rest
@@ -183,7 +184,7 @@ static void check_routes() {
         std::snprintf(buf, sizeof buf, "route heads=%d G=%d Tq=%d Tk=%d d=%d causal=%d", r.heads, r.G, r.Tq,
                       r.Tk, r.d, r.causal);
         g_case = buf;
-        const int64_t off = r.causal ? r.Tk - r.Tq : 0;
+        const int64_t off = r.off != INT32_MIN ? r.off : r.causal ? r.Tk - r.Tq : 0;
         CHECK(deep_prefill_faster(r.heads, r.G, r.Tq, r.Tk, r.d, r.causal, off, 256) == r.deep,
               "expected deep = %d", r.deep);
         CHECK(deep_prefill_faster(2 * r.heads, r.G, r.Tq, r.Tk, r.d, r.causal, off, 512) == r.deep,

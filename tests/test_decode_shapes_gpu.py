@@ -91,6 +91,17 @@ def test_decode_head_dims_above_256(nne, cuda, b, hq, hkv, d, append):
     run_case(nne, cuda, b, hq, hkv, d, lens, append, seed=hq + 3 * d)
 
 
+@pytest.mark.parametrize("hq,hkv,d,append", [(256, 8, 512, True), (264, 8, 320, True), (320, 8, 512, False)])
+def test_decode_full_units_above_256_dims(nne, cuda, hq, hkv, d, append):
+    """32 query heads or more per KV head on more (sequence, KV head) pairs than
+    CUs: full units, the deep kernel's 4-wave form (33 and 40 heads: a second
+    unit with few rows)."""
+    print("case decode deep full units hq=%d hkv=%d d=%d append=%s" % (hq, hkv, d, append), flush=True)
+    lens = np.random.default_rng(hq + d).integers(1, 70, size=33)
+    lens[7] = 130
+    run_case(nne, cuda, 33, hq, hkv, d, lens, append, seed=hq * 5 + d)
+
+
 def test_decode_long_sequences_above_256_dims(nne, cuda):
     """Few (sequence, KV head) pairs with long caches at d = 512: each head's
     keys split over workgroups, merged by the combine kernel."""

@@ -333,9 +333,8 @@ def test_stream_release_frees_and_reallocates(nne, cuda):
 ])
 def test_head_dims_above_128(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off):
     """flash_attention_forward takes any head dim (flash_attention.rs:39-48):
-    d in (128, 256] runs on the wave-pair MFMA kernel (each 32-row unit on two
-    waves, one per half of the head dim) when its work items fill the device
-    at d = 256, else on the deep kernel (its 2-wave form, or its key split for
+    d in (128, 256] runs on the 8-wave MFMA kernel when its units fill the
+    device, else on the deep kernel (its 2-wave form, or its key split for
     problems of few units), or on the split-K kernel when a KV head has at
     most 16 query rows.  (These shapes are small: all but the split-K ones
     take the deep kernel.)"""
@@ -394,12 +393,32 @@ def test_head_dims_above_256(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off):
     (2, 64, 8, 256, 256, 384, True, -10, 0),     # G = 8, rows that see no key
     (3, 24, 24, 230, 77, 448, False, 0, 1),      # Tk < Tq, a partial last unit, views
 ])
+def test_wide_kernel_257_to_512_dims(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off, layout):
+    """Prefill problems of more units than CUs (causal: more than two per CU;
+    257+ and 513+ units on the 256-CU MI355X) run the 8-wave kernel: a unit on
+    4 waves of 96 or 128 dims, K and V through one LDS buffer.  A second call
+    gives the same bits."""
+    check_twice(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off, layout)
+
+
+@pytest.mark.parametrize("b,hq,hkv,tq,tk,d,causal,q_off,layout", [
+    (1, 300, 300, 65, 65, 512, True, 0, 0),      # 3 units per KV head, a 1-row one
+    (1, 300, 300, 65, 65, 320, True, 0, 1),      # the same on [B, T, H, d] views
+    (1, 300, 300, 65, 333, 448, False, 0, 0),    # 900 units
+    (1, 257, 257, 65, 115, 260, True, 50, 0),    # a last chunk with 4 valid dims of 8, offset
+    (1, 300, 300, 65, 65, 388, True, -10, 0),    # rows that see no key
+    (1, 257, 257, 32, 300, 512, False, 0, 1),
+])
 def test_deep_four_wave_form(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off, layout):
-    """Prefill problems of more workgroups than CUs (causal: more than two
-    per CU; 257+ and 513+ units on the 256-CU MI355X) run the deep kernel's
-    4-wave form: two workgroups per CU, S from 4 partials, half of each
-    wave's Q^T in LDS.  A second call gives the same bits."""
-    print("case deep four-wave", b, hq, hkv, tq, tk, d, causal, q_off, layout, flush=True)
+    """Such problems whose KV heads have so few units that the 8-wave kernel
+    would run part empty take the deep kernel's 4-wave form: two workgroups per
+    CU, S from 4 partials, half of each wave's Q^T in LDS.  A second call gives
+    the same bits."""
+    check_twice(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off, layout)
+
+
+def check_twice(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off, layout):
+    print("case many units", b, hq, hkv, tq, tk, d, causal, q_off, layout, flush=True)
     s = 29 * tq + d
     q, k, v = rnd(s, b, hq, tq, d), rnd(s + 1, b, hkv, tk, d), rnd(s + 2, b, hkv, tk, d)
     if layout == 0:
@@ -411,14 +430,14 @@ def test_deep_four_wave_form(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off, la
     r0 = max(0, -q_off) if causal else 0
     assert not got[:, :, :r0].any()
     ref = T.ref_standard(q[:, :, r0:], k, v, causal, start_pos=q_off + r0)
-    T.assert_close(got[:, :, r0:], ref, what="d=%d four-wave" % d)
+    T.assert_close(got[:, :, r0:], ref, what="d=%d many units" % d)
 
 
 @pytest.mark.parametrize("b,hq,hkv,tq,tk,d,causal,q_off", [
     (2, 4, 4, 8, 3000, 512, False, 0),      # cross-attention: 8 queries, keys split in 8
     (1, 8, 2, 4, 2500, 384, True, 2496),    # 4 new rows at the end of a long cache, G = 4
     (1, 2, 1, 3, 1200, 1028, False, 0),     # two output chunks, each split
-    (1, 4, 4, 64, 1500, 192, False, 0),     # 129-256 dims off the wave-pair kernel: 8 units split
+    (1, 4, 4, 64, 1500, 192, False, 0),     # 129-256 dims: 8 units split
 ])
 def test_deep_key_split(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off):
     """Problems with too few query rows to fill the device split each unit's
@@ -473,16 +492,15 @@ def test_deep_head_dim_strided_views_and_repeat(nne, cuda):
     (2, 16, 16, 256, 256, 192, True, 0, 0),      # 256 units, unsplit
     (2, 16, 16, 256, 256, 192, True, 0, 1),      # the same on [B, T, H, d] views
     (2, 16, 4, 300, 350, 160, True, 50, 0),      # GQA, units straddling query heads, offset
-    (1, 32, 8, 256, 256, 256, True, 0, 0),       # d = 256 with too few wave-pair items
+    (1, 32, 8, 256, 256, 256, True, 0, 0),       # d = 256, 256 units
     (3, 8, 8, 130, 90, 228, False, 0, 0),        # Tk < Tq, a half-valid last 8-dim chunk
     (1, 4, 4, 64, 1500, 192, False, 0, 0),       # 8 units: the 8-wave key split at d = 192
 ])
 def test_deep_two_wave_form(nne, cuda, b, hq, hkv, tq, tk, d, causal, q_off, layout):
-    """Head dims 129-256 that the wave-pair kernel does not take (dims other
-    than 256, or too few of its 4-unit items to fill the device) run the deep
-    kernel: its 2-wave form, four workgroups per CU (a wave pair per 32-row
-    unit, Q^T half in LDS), or for few units its 8-wave key split.  A second
-    call gives the same bits."""
+    """Head dims 129-256 with at most as many units as CUs run the deep kernel:
+    its 2-wave form, four workgroups per CU (two waves per 32-row unit, Q^T
+    half in LDS), or for few units its 8-wave key split.  A second call gives
+    the same bits.  (The third shape has 320 units: the 8-wave MFMA kernel.)"""
     print("case deep two-wave", b, hq, hkv, tq, tk, d, causal, q_off, layout, flush=True)
     s = 31 * tq + d
     q, k, v = rnd(s, b, hq, tq, d), rnd(s + 1, b, hkv, tk, d), rnd(s + 2, b, hkv, tk, d)
@@ -513,8 +531,8 @@ def test_wide_and_deep_dims_empty_keys(nne, cuda, d):
 
 
 def test_wide_dims_kv_row_stride_beyond_deep_kernel(nne, cuda):
-    """At 129-256 dims, K/V views whose row stride is beyond the deep kernel's
-    32-bit tile offsets (2^25 floats) stay on the wave-pair kernel."""
+    """At 129-256 dims, K/V views whose row stride is beyond the 32-bit tile
+    offsets (2^25 floats) take the scalar loads of the 8-wave MFMA kernel."""
     import torch
     print("case wide dims huge kv row stride", flush=True)
     d, tk, tq = 192, 3, 40
@@ -534,14 +552,14 @@ def test_wide_dims_kv_row_stride_beyond_deep_kernel(nne, cuda):
 
 
 @pytest.mark.parametrize("b,hq,hkv,t,causal", [
-    (2, 16, 16, 1024, False),    # 256 items of 4 units: the wave-pair kernel
-    (1, 32, 8, 1024, True),      # GQA, 256 items
+    (2, 16, 16, 1024, False),    # 256 workgroups of 4 units
+    (1, 32, 8, 1024, True),      # GQA, 256 workgroups
 ])
-def test_wave_pair_kernel_full_device(nne, cuda, b, hq, hkv, t, causal):
-    """d = 256 problems whose wave-pair items fill the device stay on the
-    wave-pair kernel: sampled rows of sampled heads against the oracle, every
-    output finite."""
-    print("case wave-pair full device", b, hq, hkv, t, causal, flush=True)
+def test_wide_kernel_full_device(nne, cuda, b, hq, hkv, t, causal):
+    """d = 256 problems that fill the device with the 8-wave MFMA kernel's
+    workgroups: sampled rows of sampled heads against the oracle, every output
+    finite."""
+    print("case wide kernel full device", b, hq, hkv, t, causal, flush=True)
     d = 256
     rng = np.random.default_rng(b * hq * t + causal)
     q, k, v = (rng.standard_normal((b, h, t, d), dtype=np.float32) for h in (hq, hkv, hkv))
@@ -555,7 +573,7 @@ def test_wave_pair_kernel_full_device(nne, cuda, b, hq, hkv, t, causal):
                 ref = T.ref_standard(q[bi:bi + 1, h:h + 1, rows], k[bi:bi + 1, h // g:h // g + 1],
                                      v[bi:bi + 1, h // g:h // g + 1], causal, start_pos=r0)
                 T.assert_close(got[bi:bi + 1, h:h + 1, rows], ref,
-                               what="wave pair b %d head %d rows %d" % (bi, h, r0))
+                               what="wide b %d head %d rows %d" % (bi, h, r0))
 
 
 def test_wide_head_dim_strided_views_and_repeat(nne, cuda):

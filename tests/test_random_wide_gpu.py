@@ -2,11 +2,10 @@
 
 Each case draws a head dim in (128, 1028], a shape, a layout and a mask at
 random (numpy's generator, the case number is the seed), so the sweep crosses
-the routing of wide head dims: the wave-pair prefill kernel (d = 256 with the
-device full), the deep kernel's 2-wave form (other dims up to 256), its
-8-wave form and key split (few units), its 4-wave form (d <= 512 with more
-workgroups than CUs), its 1024-dim output chunks (d > 512) and, for decode
-steps, its ragged split.  One case in four is a large problem compared on
+the routing of wide head dims: the 8-wave MFMA kernel (up to 512 dims with more
+units than CUs), the deep kernel's 2-wave form (fewer, up to 256 dims), its
+8-wave form and key split (few units), its 1024-dim output chunks (d > 512)
+and, for decode steps, its ragged split.  One case in four is a large problem compared on
 sampled heads and rows.  References: the oracle's masked standard attention
 (llama.rs:253-296, rows without a visible key compared as zero) and its
 decode step.
@@ -27,7 +26,7 @@ def draw_case(seed):
     rng = np.random.default_rng(7000 + seed)
     d = int(rng.choice(WIDE_DIMS))
     large = seed % 4 == 3
-    if large:                                  # enough units for the 4-wave and 2-wave forms
+    if large:                                  # more units than CUs
         b = 1
         hkv = int(rng.choice([8, 16]))
         g = int(rng.choice([1, 2]))
