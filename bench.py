@@ -43,32 +43,32 @@ PEAK_HBM_GBS = 8000.0
 
 # HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE on
 # the `--probe` workload, each scaled by its reading for a plain 1 GiB device copy
-# (FETCH_SIZE x2.00, WRITE_SIZE x1.00).  Config 2 prefill: 232.9 MB read + 142.6 MB
+# (FETCH_SIZE x2.00, WRITE_SIZE x1.00).  Config 2 prefill: 234.1 MB read + 143.1 MB
 # written (algorithmic 201.3 + 134.2; part of the shared K/V is fetched into two
 # XCDs' L2).  Config 3 decode step (one launch, split heads merged inside it):
 # 646.0 MB read + 1.8 MB written (algorithmic 645.0 + 0.8, plus the partial records
 # of split heads).  Config 5b: 123.4 + 0.33 (algorithmic 123.2 + 0.33).  Config-3
 # decode prologue: 109.2 + 4.7 (algorithmic 101.2 + 0.8; partial tiles and x per
 # XCD).  GPT-2 decode attend: 104.4 + 0.3 (algorithmic 104.2 + 0.3).  Config 1:
-# 1.1 + 0.26 (algorithmic 0.79 + 0.26).  Config 4: 350.7 + 67.6 (algorithmic
+# 1.1 + 0.26 (algorithmic 0.79 + 0.26).  Config 4: 349.7 + 67.1 (algorithmic
 # 201.3 + 67.1; the persistent workgroups of a KV head on one XCD re-fetch part of
-# its 8.4 MB of K/V, more than the XCD's 4 MB L2).  Config 5a: 187.6 + 63.4
+# its 8.4 MB of K/V, more than the XCD's 4 MB L2).  Config 5a: 187.3 + 61.4
 # (algorithmic 184.3 + 61.4).  G = 8 decode step: 677.2 + 3.25 (algorithmic
 # 681.3 + 1.3, plus the 16-row partial records of split heads).  d = 256 causal
-# prefill (B = 1, H = 16, T = 4096): 297.0 + 110.6 (algorithmic 201.3 + 67.1).  d = 512
-# causal prefill (same shape): 543.0 + 165.6 (algorithmic 402.7 + 134.2;
+# prefill (B = 1, H = 16, T = 4096): 292.2 + 99.1 (algorithmic 201.3 + 67.1).  d = 512
+# causal prefill (same shape): 543.9 + 167.8 (algorithmic 402.7 + 134.2;
 # the units of a KV head re-fetch its 16.8 MB of K/V, more than the XCD's 4 MB L2).
-TRAFFIC_PREFILL_CONFIG2 = round(232.9e6 + 142.6e6)
+TRAFFIC_PREFILL_CONFIG2 = round(234.1e6 + 143.1e6)
 TRAFFIC_DECODE_CONFIG3_STEP = round(646.0e6 + 1.8e6)
 TRAFFIC_CROSS_CONFIG5B = round(123.4e6 + 0.33e6)
 TRAFFIC_PROLOGUE_CONFIG3 = round(109.2e6 + 4.7e6)
 TRAFFIC_ATTEND_GPT2 = round(104.4e6 + 0.3e6)
 TRAFFIC_PREFILL_CONFIG1 = round(1.1e6 + 0.26e6)
-TRAFFIC_PREFILL_CONFIG4 = round(350.7e6 + 67.6e6)
-TRAFFIC_PREFILL_CONFIG5A = round(187.6e6 + 63.4e6)
+TRAFFIC_PREFILL_CONFIG4 = round(349.7e6 + 67.1e6)
+TRAFFIC_PREFILL_CONFIG5A = round(187.3e6 + 61.4e6)
 TRAFFIC_DECODE_G8_STEP = round(677.2e6 + 3.25e6)
-TRAFFIC_PREFILL_D256 = round(297.0e6 + 110.6e6)
-TRAFFIC_PREFILL_D512 = round(543.0e6 + 165.6e6)
+TRAFFIC_PREFILL_D256 = round(292.2e6 + 99.1e6)
+TRAFFIC_PREFILL_D512 = round(543.9e6 + 167.8e6)
 
 
 def cpu_threads():

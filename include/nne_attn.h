@@ -121,15 +121,18 @@ int nne_counters_init(uint32_t *counters, uint64_t n, void *stream);
  * (:113).  Rows that see no key are zero (:186-194).  `o` has Q's shape.
  * Any head dim; above 128 the tensors must be 16-byte vector views
  * (d % 4 == 0, unit dim stride, other strides multiples of 4, 16-byte
- * aligned) -- NNE_EINVAL otherwise.  Above 128 dims problems with more 32-row
- * units than the device has CUs (causal above 256 dims: than two per CU) run on
- * an 8-wave kernel up to 512 dims; all others on a kernel for any head dim
- * (K/V read straight into MFMA operand layout), where problems with too few
- * query rows to fill the device split their keys over several workgroups, with
- * records in the workspace.
- * Products are those of f32 operands: each operand is the exact sum of three
- * bf16 parts on the bf16 matrix cores, or taken whole on the f32 ones, and all
- * sums are f32. */
+ * aligned) -- NNE_EINVAL otherwise.  Above 128 dims most problems with more
+ * 32-row units than the device has CUs (causal above 256 dims: than two per CU)
+ * run on an 8-wave kernel up to 512 dims; the others (KV heads of few units,
+ * and larger dims) on a kernel for any head dim (K/V read straight into MFMA
+ * operand layout), where problems with too few query rows to fill the device
+ * split their keys over several workgroups, with records in the workspace.
+ * Products are those of f32 operands: each operand is the sum of three bf16
+ * parts on the bf16 matrix cores (exact; of a key below 2^-110 to 2^-134), or
+ * taken whole on the f32 ones, and all sums are f32.  32 query rows whose values
+ * the parts cannot hold (a result that is not finite; queries times the scale
+ * beyond 2^90 or, not zero, below 2^-110) are computed again with f32 products,
+ * at two to three times the time. */
 int nne_flash_attention_forward(const float *q, const int64_t q_shape[4], const int64_t q_strides[4],
                                 const float *k, const int64_t k_shape[4], const int64_t k_strides[4],
                                 const float *v, const int64_t v_shape[4], const int64_t v_strides[4],

@@ -1,7 +1,8 @@
 // Attention at head dims above 256: prefill, cross-attention and decode over a
 // KV cache, on v_mfma_f32_32x32x2_f32; and prefill at 129-256 dims.  Prefill up
-// to 512 dims with more 32-row units than CUs (above 256 dims, causal: than two
-// per CU) runs on prefill_wide_kernel instead, on the bf16 matrix cores.
+// to 512 dims runs on prefill_wide_kernel, on the bf16 matrix cores, where that
+// one is estimated to be no slower (deep_prefill_faster: most calls of more
+// 32-row units than CUs, above 256 dims, causal: than two per CU).
 //
 // Algorithm: the online softmax of the reference's flash_attention_forward
 // (src/nn/flash_attention.rs:91-195) over 32-key tiles, rows that see no key
@@ -36,8 +37,8 @@
 //  * The next tile's K (up to 8 chunks) is loaded during the current tile's
 //    exchange, softmax and P V, and a tile's V at its start, under its S.
 //  Up to 512 dims, full units on more workgroups than CUs (those that
-//  prefill_wide_kernel does not take: decode steps of 32 query heads or more
-//  per KV head, K/V row strides beyond that kernel's) use a 4-wave form
+//  prefill_wide_kernel does not take: KV heads of few units, and decode steps
+//  of 32 query heads or more per KV head) use a 4-wave form
 //  instead, two workgroups per CU: each wave takes twice the chunks and
 //  output blocks (S from 4 partials, Q^T of its last 8 chunks in LDS), so a
 //  tile's MFMAs per wave double against the same exchange and softmax, and
@@ -196,8 +197,8 @@ __global__ __launch_bounds__(64 * DW, DW == 8 ? 1 : 2) void deep_attention_kerne
     // other rows, at no weight), so no load needs a predicate and the byte
     // offsets are a lane constant plus a small uniform part.  K columns past d
     // (the odd half of a last 8-dim chunk when d % 8 == 4) are read from memory
-    // next to the row and zeroed; V columns past d read
-    // the row's last float and only reach O columns never stored.
+    // next to the row and zeroed; V columns past d read the row's last float and
+    // only reach O columns never stored.
     auto range = [&](const float* base, int64_t st, int key0) {
         const int nk = kend - key0 < 32 ? kend - key0 : 32;
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + key0 * st), 0,
@@ -605,7 +606,7 @@ hipError_t launch_deep_v(DeepParams p, hipStream_t stream) {
 // long one runs alone with one wave per SIMD), and so do decode steps (a few
 // rows per unit, streaming their caches: B = 32, d = 512 634 us with 8
 // waves, 781 us with 4).
-// Head dims 129-256 (prefill with at most as many 32-row units as CUs) run the
+// Head dims 129-256 (the prefill that deep_prefill_faster sends here) run the
 // 2-wave form unsplit, and the 8-wave form's key split.
 template <bool CAUSAL>
 hipError_t launch_deep_t(const DeepParams& p, int cus, hipStream_t stream) {

@@ -41,9 +41,9 @@
 // (softmax, the parts of P, K and V); with random operands a stream of nothing
 // but these MFMAs settles at 1777 TFLOP/s, 296 TFLOP/s of f32 products.
 // Measured against the f32 MFMAs (v_mfma_f32_32x32x2, 157 TFLOP/s at most):
-// B = 4, Hq = 32, Hkv = 8, T = 2048, d = 128 causal 1067 -> 742 us, B = 1,
-// H = 16, T = 16384, d = 64 causal 4300 -> 2800 us, B = 8, H = 20, T = 1500,
-// d = 64 774 -> 475 us, with 0.6 to 0.9 of the error against 64 bits.
+// B = 4, Hq = 32, Hkv = 8, T = 2048, d = 128 causal 1075 -> 697-717 us, B =
+// 1, H = 16, T = 16384, d = 64 causal 4346 -> 2810-2970 us, B = 8, H = 20, T =
+// 1500, d = 64 777 -> 484 us, with 0.4 to 0.9 of the error against 64 bits.
 //
 // Problems with fewer work items than CUs instead cut each item's key tiles
 // into chunks, one workgroup per (item, chunk); the last chunk of an item to
@@ -197,7 +197,7 @@ struct SplitTile {
                     kr[i] = __builtin_bit_cast(
                         float4, __builtin_amdgcn_raw_buffer_load_b128(range, k_lane[i % NC], i / NC * k_step, 0));
             } else {
-                // The range check is on the lane's offset, so all of it goes there.
+                // (Whole offsets in the lanes: the check of the tail's rows takes in no other.)
 #pragma unroll
                 for (int i = 0; i < NK; ++i)
                     kr[i] = __builtin_bit_cast(
@@ -519,8 +519,9 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
     // -- t on their first (long) items, total - t on their second (short)
     // ones, whatever their ranks -- so the head's K/V tiles they read stay in
     // the XCD's L2.  Walked forwards, every second item restarts at key 0 at
-    // its own time and the walks spread over the whole head: config 4 read
-    // 284 MB from HBM, 249 MB backwards (201 MB algorithmic); same time.
+    // its own time and the walks spread over the whole head: B = 1, H = 16, T =
+    // 16384, d = 64 read 284 MB from HBM, 249 MB backwards on the f32 MFMAs (201 MB
+    // algorithmic), same time; 350 MB now.
     const bool rev = !SPLIT && p.pairing && (j & 1);
     const int kstep = rev ? -1 : 1;
     const int kfirst = rev ? t1 - 1 : t0;
@@ -852,12 +853,11 @@ __global__ __launch_bounds__(256, D >= 128 && !VEC ? 1 : D <= 64 && !SPLIT ? 3 :
 // What bounds it: the barriers.  The waves of a CU run their MFMAs and their
 // softmax at the same time; up to 256 dims the parts of K and V are therefore
 // computed between the MFMAs of the same wave (d = 256, T = 4096 820 -> 785 us,
-// d = 192 1830 -> 1690 us).  The matrix cores are busy 51 % of the cycles at 256
-// dims without that and 37 % at 512 (a staged tile serves only 64 rows there: 630
-// vector instructions beside 96 MFMAs per wave and tile).  Against the f32 MFMAs:
-// B = 1, H = 16, T = 4096 causal, d = 256 1190 -> 780 us, d = 512 2410 -> 1930 us;
-// B = 8, H = 20, T = 1500, d = 192 2570 -> 1690 us, at 0.6 to 0.7 of the error
-// against 64 bits.
+// d = 192 1830 -> 1690 us).  The matrix cores are busy 48 % of the cycles at 256
+// dims and 34 % at 512 (a staged tile serves only 64 rows there: 8 vector
+// instructions per MFMA).  Against the f32 MFMAs: B = 1, H = 16, T = 4096 causal,
+// d = 256 1204 -> 775 us, d = 512 2412 -> 1964 us; B = 8, H = 20, T = 1500, d = 192
+// 2570 -> 1675 us, at 0.6 to 0.7 of the error against 64 bits.
 template <int DW, int NW, bool CAUSAL, bool VEC>
 __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParams p) {
     constexpr int D = DW * NW, U = 8 / NW;
@@ -952,7 +952,7 @@ __global__ __launch_bounds__(512, 1) void prefill_wide_kernel(const PrefillParam
 
     // Second items of causal pairs walk their key tiles backwards, as in the
     // d <= 128 kernel (a head's K/V tiles stay in the XCD's L2: 688 -> 260 MB
-    // read at B = 1, H = 16, T = 4096, d = 256).
+    // read at B = 1, H = 16, T = 4096, d = 256 on the f32 MFMAs; 292 now).
     const bool rev = p.pairing && (j & 1);
     const int kstep = rev ? -1 : 1;
     const int kfirst = rev ? n_tiles - 1 : 0;
